@@ -11,6 +11,8 @@
 namespace mcr {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define MCR_CONSTP(T) const __attribute__((address_space(4))) T*
 
@@ -213,8 +215,10 @@ __device__ __forceinline__ uint16_t bf16_bits(float f) {
 __device__ __forceinline__ float bf16_val(uint16_t b) { return as_f32((uint32_t)b << 16); }
 
 
+// Converted as a vector: one v_cvt_pk_bf16_f32 (two scalar conversions and
+// their merge were four instructions).
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)bf16_bits(lo) | ((uint32_t)bf16_bits(hi) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
 // z[0..7] -> bf16 hi and lo parts, two per 32-bit word

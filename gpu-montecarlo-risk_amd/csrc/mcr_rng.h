@@ -50,23 +50,58 @@ MCR_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
 #endif
 }
 
-MCR_HD Ctr4 philox4x32_10(Ctr4 c, uint32_t k0, uint32_t k1) {
+struct Key2 {
+  uint32_t k0, k1;
+};
+MCR_HD Key2 key_of(uint64_t seed) { return Key2{(uint32_t)seed, (uint32_t)(seed >> 32)}; }
+
+// Rounds R0 .. 9 of the ten.
+template <int R0>
+MCR_HD Ctr4 philox_rounds(Ctr4 c, Key2 k) {
+  uint32_t k0 = k.k0 + R0 * kPhiloxW0, k1 = k.k1 + R0 * kPhiloxW1;
 #pragma unroll
-  for (int r = 0; r < 10; ++r) {
-    if (r) {
-      k0 += kPhiloxW0;
-      k1 += kPhiloxW1;
-    }
+  for (int r = R0; r < 10; ++r) {
     const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
     const uint64_t p1 = (uint64_t)kPhiloxM1 * c.z;
-    Ctr4 n;
-    n.x = xor3((uint32_t)(p1 >> 32), c.y, k0);
-    n.y = (uint32_t)p1;
-    n.z = xor3((uint32_t)(p0 >> 32), c.w, k1);
-    n.w = (uint32_t)p0;
-    c = n;
+    c = Ctr4{xor3((uint32_t)(p1 >> 32), c.y, k0), (uint32_t)p1, xor3((uint32_t)(p0 >> 32), c.w, k1),
+             (uint32_t)p0};
+    k0 += kPhiloxW0;
+    k1 += kPhiloxW1;
   }
   return c;
+}
+MCR_HD Ctr4 philox4x32_10(Ctr4 c, uint32_t k0, uint32_t k1) {
+  return philox_rounds<0>(c, Key2{k0, k1});
+}
+
+// Counter (block, 0, path lo, path hi): the first two of the ten rounds hold
+// products of the path's low word alone (once per path) and products of the
+// block and the path's high word alone.  Kernels whose block index and path
+// high word are uniform over a wave get the latter from the scalar unit, which
+// leaves 16 of the 20 64-bit products of a block to the vector unit.
+struct PhiloxPath {
+  uint32_t y1;      // round 1: y
+  uint32_t zh, w2;  // round 2: z before the block's part, w
+};
+struct PhiloxBlock {
+  uint32_t x2, y2, zb;  // round 2: x before the path's part, y, the block's part of z
+};
+
+MCR_HD PhiloxPath philox_path(uint32_t path_lo, Key2 k) {
+  const uint64_t p1 = (uint64_t)kPhiloxM1 * path_lo;
+  const uint64_t p0 = (uint64_t)kPhiloxM0 * ((uint32_t)(p1 >> 32) ^ k.k0);
+  return PhiloxPath{(uint32_t)p1, (uint32_t)(p0 >> 32), (uint32_t)p0};
+}
+
+MCR_HD PhiloxBlock philox_block(uint32_t blk, uint32_t path_hi, Key2 k) {
+  const uint64_t p0 = (uint64_t)kPhiloxM0 * blk;
+  const uint64_t p1 = (uint64_t)kPhiloxM1 * ((uint32_t)(p0 >> 32) ^ path_hi ^ k.k1);
+  return PhiloxBlock{(uint32_t)(p1 >> 32) ^ (k.k0 + kPhiloxW0), (uint32_t)p1,
+                     (uint32_t)p0 ^ (k.k1 + kPhiloxW1)};
+}
+
+MCR_HD Ctr4 philox4x32_10(PhiloxPath p, PhiloxBlock b, Key2 k) {
+  return philox_rounds<2>(Ctr4{p.y1 ^ b.x2, b.y2, p.zh ^ b.zb, p.w2}, k);
 }
 
 MCR_HD float as_f32(uint32_t b) { return __builtin_bit_cast(float, b); }
@@ -96,14 +131,28 @@ constexpr float kCos2 = 0x1.03c1dep+6f;
 constexpr float kCos3 = -0x1.55c664p+6f;
 constexpr float kCos4 = 0x1.d9f7bep+5f;
 
-// -ln(u) for u = ((a >> 8) + 1) * 2^-24.  Range reduction u = 2^e m with
+// The transform below computes the stream definition's r and theta with as few
+// instructions as give the same bits (a Box-Muller pair takes 49 VALU
+// instructions against 56 for the plain form; checked on the host over all
+// 2^24 logarithm inputs and all 2^32 angles.  With the packed bf16 conversion
+// of the path kernels a query of n = 50, 1e8 paths went from 5.71 to 5.11 ms):
+//  - the exponent of u stays in place, as e * 2^23, so that subtracting it from
+//    the bit pattern gives the mantissa and converting it gives e scaled by a
+//    power of two, which the ln 2 constants take back;
+//  - the logarithm keeps its sign (l = ln u <= 0): the root reads -l = h through
+//    its seed constant and the sign of its Newton product;
+//  - the root's factor 2 sits in the sine and cosine coefficients (powers of
+//    two commute with rounding);
+//  - the quarter turn's sign goes onto the radius, once for both results, and
+//    its parity is read as a float compare.
+
+// ln(u) for u = ((a >> 8) + 1) * 2^-24.  Range reduction u = 2^e m with
 // m in [sqrt(1/2), sqrt(2)) done on the fp32 bit pattern.
-MCR_HD float neg_log_u24(uint32_t a) {
+MCR_HD float log_u24(uint32_t a) {
   const float u = __builtin_fmaf((float)(a >> 8), 0x1p-24f, 0x1p-24f);  // exact
-  const int32_t ix = (int32_t)as_u32(u) - 0x3f3504f3;
-  const int32_t e = ix >> 23;
-  const float m = as_f32((uint32_t)(ix & 0x007fffff) + 0x3f3504f3u);
-  const float f = m - 1.0f;  // exact (Sterbenz)
+  const uint32_t ub = as_u32(u);
+  const uint32_t eh = (ub - 0x3f3504f3u) & 0xff800000u;  // e * 2^23
+  const float f = as_f32(ub - eh) - 1.0f;                // m - 1, exact (Sterbenz)
   float p = kLogP6;
   p = __builtin_fmaf(p, f, kLogP5);
   p = __builtin_fmaf(p, f, kLogP4);
@@ -114,75 +163,77 @@ MCR_HD float neg_log_u24(uint32_t a) {
   const float q = __builtin_fmaf(p, f, -0.5f);
   const float t = f * f;
   const float l1p = __builtin_fmaf(t, q, f);
-  const float ef = (float)e;
-  const float lo = __builtin_fmaf(ef, kLn2Lo, l1p);
-  return -__builtin_fmaf(ef, kLn2Hi, lo);
+  const float ef = (float)(int32_t)eh;
+  const float lo = __builtin_fmaf(ef, kLn2Lo * 0x1p-23f, l1p);
+  return __builtin_fmaf(ef, kLn2Hi * 0x1p-23f, lo);
 }
 
-// sqrt(2 h) for h in [0, 17]: bit-pattern seed for 1/sqrt(2h) (Lomont's
-// constant 0x5f375a86 with the factor 2 folded into the exponent; 3.4% worst
-// error), three Newton steps g <- g (3/2 - h g^2) (error 1.7e-3, 4.6e-6, then
-// fp32 rounding), then 2h * g.  The iteration runs on hn = h + 2^-60, which
-// equals h for every nonzero h here (h >= 5.9e-8) and keeps g finite at h = 0,
-// where the result is 0.
-MCR_HD float sqrt_twice(float h) {
-  const float hn = h + 0x1p-60f;
-  float g = as_f32(0x5ef75a86u - (as_u32(hn) >> 1));
+// sqrt(2 h) / 2 for l = -h, h in [0, 17]: bit-pattern seed for 1/sqrt(2h)
+// (Lomont's constant 0x5f375a86 with the factor 2 folded into the exponent and
+// the sign bit of l, which the shift brings down, taken out; 3.4% worst error),
+// three Newton steps g <- g (3/2 - h g^2) (error 1.7e-3, 4.6e-6, then fp32
+// rounding), then h * g.  At h = 0 (l = +0) the seed is a tiny negative number,
+// the iteration keeps it finite and the result is -0.
+MCR_HD float half_sqrt_twice(float l) {
+  float g = as_f32(0x9ef75a86u - (as_u32(l) >> 1));
 #pragma unroll
   for (int it = 0; it < 3; ++it) {
     float t = g * g;
-    t = __builtin_fmaf(-hn, t, 1.5f);
+    t = __builtin_fmaf(l, t, 1.5f);
     g = g * t;
   }
-  return (h + h) * g;
+  return __builtin_fabsf(l) * g;
 }
 
-// cos and sin of 2*pi*b/2^32.  The nearest quarter turn q comes from the top
-// bits of b, the signed remainder (30 bits) is the reduced argument in turns.
-MCR_HD void sincos_turn(uint32_t b, float* c_out, float* s_out) {
+// (r cos theta, r sin theta) for theta = 2 pi b / 2^32 and hr = r / 2.  The
+// nearest quarter turn q comes from the top bits of b, the signed remainder (30
+// bits) is the reduced argument in turns; s and c below are twice its sine and
+// cosine.
+MCR_HD void rotate_turn(uint32_t b, float hr, float* z0, float* z1) {
   const int32_t rem = (int32_t)(b << 2) >> 2;
-  const uint32_t q = (b - (uint32_t)rem) >> 30;
+  uint32_t q = b - (uint32_t)rem;  // quarter turns, in bits 30 and 31
+#if defined(__HIP_DEVICE_COMPILE__)
+  // opaque, or the compare below becomes a mask and an integer compare
+  asm("" : "+v"(q));
+#endif
   const float a = (float)rem * 0x1p-32f;
   const float t = a * a;
-  float s = __builtin_fmaf(kSin3, t, kSin2);
-  s = __builtin_fmaf(s, t, kSin1);
-  s = __builtin_fmaf(s, t, kSin0);
+  float s = __builtin_fmaf(2.0f * kSin3, t, 2.0f * kSin2);
+  s = __builtin_fmaf(s, t, 2.0f * kSin1);
+  s = __builtin_fmaf(s, t, 2.0f * kSin0);
   s = s * a;
-  float c = __builtin_fmaf(kCos4, t, kCos3);
-  c = __builtin_fmaf(c, t, kCos2);
-  c = __builtin_fmaf(c, t, kCos1);
-  c = __builtin_fmaf(c, t, 1.0f);
-  const float sw_s = (q & 1u) ? c : s;
-  const float sw_c = (q & 1u) ? s : c;
-  *s_out = as_f32(as_u32(sw_s) ^ ((q & 2u) << 30));
-  *c_out = as_f32(as_u32(sw_c) ^ (((q + 1u) & 2u) << 30));
+  float c = __builtin_fmaf(2.0f * kCos4, t, 2.0f * kCos3);
+  c = __builtin_fmaf(c, t, 2.0f * kCos2);
+  c = __builtin_fmaf(c, t, 2.0f * kCos1);
+  c = __builtin_fmaf(c, t, 2.0f);
+  const float w = as_f32(as_u32(hr) ^ (q & 0x80000000u));
+  const bool odd = as_f32(q) != 0.0f;  // 2.0 or -2.0, against 0.0 and -0.0
+  *z0 = w * (odd ? -s : c);
+  *z1 = w * (odd ? c : s);
 }
 
 MCR_HD void box_muller(uint32_t a, uint32_t b, float* z0, float* z1) {
-  const float r = sqrt_twice(neg_log_u24(a));
-  float c, s;
-  sincos_turn(b, &c, &s);
-  *z0 = r * c;
-  *z1 = r * s;
+  rotate_turn(b, half_sqrt_twice(log_u24(a)), z0, z1);
 }
 
-struct Key2 {
-  uint32_t k0, k1;
-};
-MCR_HD Key2 key_of(uint64_t seed) { return Key2{(uint32_t)seed, (uint32_t)(seed >> 32)}; }
-
 // Normals z[4*blk .. 4*blk+3] of one path.
-MCR_HD void normals4(Key2 key, uint64_t path, uint32_t blk, float z[4]) {
-  const Ctr4 x = philox4x32_10(Ctr4{blk, 0u, (uint32_t)path, (uint32_t)(path >> 32)}, key.k0, key.k1);
+MCR_HD void normals4(Key2 key, PhiloxPath path, PhiloxBlock blk, float z[4]) {
+  const Ctr4 x = philox4x32_10(path, blk, key);
   box_muller(x.x, x.y, &z[0], &z[1]);
   box_muller(x.z, x.w, &z[2], &z[3]);
+}
+MCR_HD void normals4(Key2 key, uint64_t path, uint32_t blk, float z[4]) {
+  normals4(key, philox_path((uint32_t)path, key), philox_block(blk, (uint32_t)(path >> 32), key), z);
 }
 
 // normals4's z[0], z[1] alone (the same bits): for a path's last block when
 // n leaves its second pair unused.
-MCR_HD void normals2(Key2 key, uint64_t path, uint32_t blk, float z[2]) {
-  const Ctr4 x = philox4x32_10(Ctr4{blk, 0u, (uint32_t)path, (uint32_t)(path >> 32)}, key.k0, key.k1);
+MCR_HD void normals2(Key2 key, PhiloxPath path, PhiloxBlock blk, float z[2]) {
+  const Ctr4 x = philox4x32_10(path, blk, key);
   box_muller(x.x, x.y, &z[0], &z[1]);
+}
+MCR_HD void normals2(Key2 key, uint64_t path, uint32_t blk, float z[2]) {
+  normals2(key, philox_path((uint32_t)path, key), philox_block(blk, (uint32_t)(path >> 32), key), z);
 }
 
 }  // namespace mcr
