@@ -70,7 +70,12 @@ __device__ __forceinline__ void append_loss(const PathArgs& a, int al, bool in, 
   if (m == 0ull) return;
   const int lane = __lane_id();
   const int leader = __ffsll((long long)m) - 1;
-  const unsigned rank = __popcll(m & ((1ull << lane) - 1ull));
+  // set bits of m below this lane, counted by mbcnt: the mask by a 64-bit shift
+  // gave wrong ranks where the compiler had put the lane index, its shift
+  // amount, into the last register of the wave's allocation (two losses of a
+  // wave then shared a slot)
+  const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
   unsigned long long base = 0;
   if (lane == leader) base = atomicAdd(&a.acc->gathered[al], (unsigned long long)__popcll(m));
   base = __shfl(base, leader);
