@@ -2,6 +2,7 @@
 // C-ABI implementation (mcr_api.cpp).  Not part of the public ABI.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace mcr {
@@ -50,6 +51,11 @@ struct DevAccum {
   unsigned long long hist_below;            // refinement: losses < hist_lo
   unsigned long long hist_above;            // refinement: losses past the last bin
 };
+// (flush_tally_lds addresses its words in this order)
+static_assert(offsetof(DevAccum, near) == 8 && offsetof(DevAccum, above) == 16 &&
+                  offsetof(DevAccum, sum_above) == 16 + 8 * kMaxAlpha &&
+                  offsetof(DevAccum, hist_above) == offsetof(DevAccum, hist_below) + 8,
+              "flush_tally_lds");
 
 // Kernel arguments (passed by value).
 struct PathArgs {

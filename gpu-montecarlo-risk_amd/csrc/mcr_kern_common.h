@@ -152,6 +152,66 @@ __device__ __forceinline__ void flush_tally(const PathArgs& a, const LaneTally& 
   }
 }
 
+// The same tallies for kernels whose waves finish 64 paths at once: kept in LDS
+// (ballots and population counts, added by one lane; the few losses above a
+// window add themselves), so a path loop carries none of them in registers.
+// One record per flushing unit (a workgroup, or a wave of the batch kernels).
+struct LdsTally {
+  unsigned long long v[4 + 2 * kMaxAlpha];  // count, near, hist below / above,
+                                            // above[], sum_above[]
+};
+constexpr int kTallyWords = 4 + 2 * kMaxAlpha;
+
+// All 64 lanes of the wave, valid marking the paths that count.
+__device__ __forceinline__ void tally_wave(const PathArgs& a, LdsTally* t, uint64_t q, bool valid,
+                                           int S, float loss, bool near, unsigned* sh_hist) {
+  const DevInfo* ip = a.info;
+  asm volatile("" : "+s"(ip));
+  MCR_CONSTP(DevInfo) w = cview(ip);
+  auto add = [&](int slot, bool on) {
+    const unsigned long long m = __ballot(on);
+    if (m != 0ull && __lane_id() == 0) atomicAdd(&t->v[slot], (unsigned long long)__popcll(m));
+  };
+  add(0, valid && S >= a.k);
+  if (a.thr_lo < a.thr_hi) add(1, valid && near);
+  if (valid) {
+    if (a.S_out) a.S_out[q] = S;
+    if (a.loss_out) a.loss_out[q] = loss;
+    if (sh_hist) atomicAdd(&sh_hist[S], 1u);
+  }
+  if (a.loss_mode == kLossBracket) {
+#pragma unroll
+    for (int al = 0; al < kMaxAlpha; ++al) {
+      if (al < a.n_alpha) {
+        const bool above = valid && loss > w->hi[al];
+        add(4 + al, above);
+        if (above) atomicAdd(&t->v[4 + kMaxAlpha + al], (unsigned long long)fixed32(loss));
+        append_loss(a, al, valid && loss >= w->lo[al] && loss <= w->hi[al], loss);
+      }
+    }
+  } else if (a.loss_mode == kLossHist) {
+    const float pos = (loss - w->hist_lo) * w->hist_scale;
+    const bool below = !(pos >= 0.0f);  // also catches NaN
+    const bool past = !below && !(pos < (float)kHistBins);
+    add(2, valid && below);
+    add(3, valid && past);
+    if (valid && !below && !past) atomicAdd(&a.hist[(int)pos], 1u);
+  }
+}
+
+// Lane i of the first 12 adds word i to the query's accumulators and clears it.
+__device__ __forceinline__ void flush_tally_lds(const PathArgs& a, LdsTally* t, int i) {
+  if (i >= kTallyWords) return;
+  unsigned long long* const acc = &a.acc->count;
+  // DevAccum: count, near, above[], sum_above[], gathered[], hist below, hist above
+  unsigned long long* dst = i < 2 ? acc + i
+                            : i < 4 ? &a.acc->hist_below + (i - 2)
+                                    : acc + (i - 2);
+  const unsigned long long v = t->v[i];
+  t->v[i] = 0ull;
+  if (v) atomicAdd(dst, v);
+}
+
 // Workgroup form of flush_tally for kernels whose waves all tally paths: each
 // wave sums its lanes, the waves' sums meet in LDS, and wave 0 issues one
 // atomic per counter for the whole workgroup (a per-wave flush costs every
@@ -226,15 +286,17 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
+// z0, z1 -> their bf16 hi and lo parts, two per 32-bit word
+__device__ __forceinline__ void split2(float z0, float z1, uint32_t* hi, uint32_t* lo) {
+  const uint32_t h = pack_bf16x2(z0, z1);
+  *hi = h;
+  *lo = pack_bf16x2(z0 - as_f32(h << 16), z1 - as_f32(h & 0xffff0000u));
+}
+
 // z[0..7] -> bf16 hi and lo parts, two per 32-bit word
 __device__ __forceinline__ void split8(const float* z, uint32_t hi[4], uint32_t lo[4]) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    hi[q] = pack_bf16x2(z[2 * q], z[2 * q + 1]);
-    const float r0 = z[2 * q] - as_f32(hi[q] << 16);
-    const float r1 = z[2 * q + 1] - as_f32(hi[q] & 0xffff0000u);
-    lo[q] = pack_bf16x2(r0, r1);
-  }
+  for (int q = 0; q < 4; ++q) split2(z[2 * q], z[2 * q + 1], &hi[q], &lo[q]);
 }
 
 // lanes 32-63 of x <-> lanes 0-31 of y
@@ -242,6 +304,12 @@ __device__ __forceinline__ void swap32(uint32_t& x, uint32_t& y) {
   const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
   x = r[0];
   y = r[1];
+}
+__device__ __forceinline__ void swap32(float& x, float& y) {
+  uint32_t u = as_u32(x), v = as_u32(y);
+  swap32(u, v);
+  x = as_f32(u);
+  y = as_f32(v);
 }
 
 __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t w[4]) {

@@ -12,8 +12,8 @@ namespace mcr {
 // and l + 32 share path l % 32, generating its normals 16s..16s+7 and
 // 16s+8..16s+15 of each step s: their B-operand slots.  D[row][path]: lane l
 // holds rows 8(r/4) + 4(l/32) + r%4 of its path; one v_permlane32_swap sums
-// the two halves' crash counts, and the upper lane, which holds the loss row,
-// tallies the path.
+// the two halves' crash counts, and once both tiles are done another brings the
+// losses (row 32T-1, in the upper lanes) to one lane per path for the tally.
 // ---------------------------------------------------------------------------
 // NB = Philox blocks per path (n <= 4 NB), T = row tiles; both compile-time
 // so every block, step and tile bound below is a constant.
@@ -25,7 +25,7 @@ namespace mcr {
 // normals need no lane exchange and the half-wave pair shares one path.
 template <int NB, int T>
 __device__ __forceinline__ void mfma_wave_groups(const PathArgs& a, uint64_t g0, uint64_t g1,
-                                                 uint64_t gstep, LaneTally& t, unsigned* sh_hist) {
+                                                 uint64_t gstep, LdsTally* t, unsigned* sh_hist) {
   constexpr int S = (NB + 3) / 4;  // 16-wide K steps
   const int lane = threadIdx.x & 63;
   const int h = lane >> 5;
@@ -38,10 +38,11 @@ __device__ __forceinline__ void mfma_wave_groups(const PathArgs& a, uint64_t g0,
   const float4* __restrict__ rinit = (const float4*)a.rowinit;
 
   for (uint64_t grp = g0; grp < g1; grp += gstep) {
+    uint32_t S0 = 0, S1 = 0;
+    float loss0 = 0.0f, loss1 = 0.0f;
 #pragma unroll 1
     for (int sub = 0; sub < 2; ++sub) {
-      const uint64_t q = grp * 64 + 32 * sub + (lane & 31);
-      const uint64_t path = a.path0 + q;
+      const uint64_t path = a.path0 + grp * 64 + 32 * sub + (lane & 31);
       f32x16 acc[T];
 #pragma unroll
       for (int s = 0; s < S; ++s) {
@@ -107,30 +108,43 @@ __device__ __forceinline__ void mfma_wave_groups(const PathArgs& a, uint64_t g0,
         }
       uint32_t c2 = c;
       swap32(c, c2);  // c = the lower half's counts, c2 = the upper half's, in every lane
-      const int Sp = (int)(c + c2);
-      const float loss = acc[T - 1][15];  // row 32T - 1 in the upper half-wave
-      if (h == 1 && q < a.npaths) tally_path(a, t, q, Sp, loss, false, sh_hist);
+      S0 = S1;
+      loss0 = loss1;
+      S1 = c + c2;
+      loss1 = acc[T - 1][15];  // row 32T - 1 in the upper half-wave
     }
+    swap32(loss0, loss1);  // loss1 = tile 0's losses below, tile 1's above
+    const uint64_t q = grp * 64 + lane;
+    tally_wave(a, t, q, q < a.npaths, (int)(h ? S1 : S0), loss1, false, sh_hist);
   }
 }
 
+// Waves per SIMD the register budget must allow.  The kernel is bound by VALU
+// issue, which pairs instructions of two waves: an odd number of waves leaves
+// one without a partner (three waves generate normals no faster than two), so
+// the budget is that of four waves, or of two where the accumulators of 3 or 4
+// tiles leave no room.  Measured at 4e11 / (n^2 + 40 n) paths: T = 1 with 8 or
+// 6 waves n = 31 6.43 / 4.80 ms against 4.82; T = 2 with 5 n = 50 5.27 against
+// 4.32; T = 3, 4 with 3 or 4 waves spill (n = 110 5.31 / 4.80 against 2.90).
+constexpr int mfma_min_waves(int T) { return T <= 2 ? 4 : 2; }
+
 template <int NB, int T>
-__global__ __launch_bounds__(256) void k_mfma(PathArgs a) {
+__global__ __launch_bounds__(256, mfma_min_waves(T)) void k_mfma(PathArgs a) {
   __shared__ unsigned sh_hist[32 * kMfmaMaxT];
+  __shared__ LdsTally t;
   const int n = a.n;
   const bool want_hist = a.s_hist != nullptr;
   if (want_hist) {
     for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
-    __syncthreads();
   }
-  LaneTally t;
-  zero_tally(t);
+  if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
+  __syncthreads();
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x >> 6);
   mfma_wave_groups<NB, T>(a, (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6),
-                          (a.npaths + 63) / 64, waves, t, want_hist ? sh_hist : nullptr);
-  flush_tally_block(a, t);
+                          (a.npaths + 63) / 64, waves, &t, want_hist ? sh_hist : nullptr);
+  __syncthreads();
+  flush_tally_lds(a, &t, threadIdx.x);
   if (want_hist) {
-    __syncthreads();
     for (int i = threadIdx.x; i <= n; i += blockDim.x)
       if (sh_hist[i]) atomicAdd(&a.s_hist[i], (unsigned long long)sh_hist[i]);
   }
@@ -141,18 +155,20 @@ __global__ __launch_bounds__(256) void k_mfma(PathArgs a) {
 // the list is exhausted, and flushes its tally into the item's query after
 // each item.  Waves never wait for each other.
 template <int NB, int T>
-__global__ __launch_bounds__(256) void k_batch_small(BatchArgs b) {
+__global__ __launch_bounds__(256, mfma_min_waves(T)) void k_batch_small(BatchArgs b) {
+  __shared__ LdsTally tally[4];
+  const int lane = threadIdx.x & 63;
+  LdsTally* t = &tally[threadIdx.x >> 6];
+  if (lane < kTallyWords) t->v[lane] = 0ull;
   for (;;) {
     unsigned it = 0;
-    if ((threadIdx.x & 63) == 0) it = atomicAdd(b.next, 1u);
+    if (lane == 0) it = atomicAdd(b.next, 1u);
     it = __builtin_amdgcn_readfirstlane(it);  // lane 0 took the item for the wave
     if (it >= b.nitems) break;
     const WorkItem w = load_const(b.items + it);
     const PathArgs a = load_const(b.qs + w.query);
-    LaneTally t;
-    zero_tally(t);
     mfma_wave_groups<NB, T>(a, w.first_group, w.first_group + w.ngroups, 1, t, nullptr);
-    flush_tally(a, t);
+    flush_tally_lds(a, t, lane);
   }
 }
 
