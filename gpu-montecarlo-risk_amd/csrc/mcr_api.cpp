@@ -186,6 +186,7 @@ struct DevBuffers {
 
 struct Plan {
   int n, T, S, r8;
+  bool f32;  // fp32 fragments (S octets) in lfrag
   int kernel;
   int n_alpha;
   bool per_path;
@@ -206,7 +207,7 @@ size_t layout(const Plan& p, char* base, DevBuffers* b) {
   b->L32 = c.take<float>((size_t)p.r8 * p.r8);
   b->mu32 = c.take<float>(n);
   b->v32 = c.take<float>(n);
-  b->lfrag = c.take<uint4>((size_t)p.T * p.S * 64 * 2);
+  b->lfrag = c.take<uint4>((size_t)p.T * p.S * 64 * (p.f32 ? 1 : 2));
   b->rowinit = c.take<float>((size_t)32 * p.T);
   b->gather = c.take<float>((size_t)std::max(p.n_alpha, 1) * kGatherCap);
   b->hist = c.take<unsigned>(kHistBins);
@@ -269,12 +270,16 @@ int choose_kernel(const mcr_query* q, Plan* p) {
     return MCR_E_UNSUPPORTED;
   }
   p->kernel = k;
+  p->T = p->S = 0;
+  p->f32 = false;
   if (k == MCR_KERNEL_MFMA || k == MCR_KERNEL_MFMA_LDS) {
     p->T = (n + 1 + 31) / 32;
     p->S = (n + 15) / 16;
-  } else {
-    p->T = 0;
-    p->S = 0;
+  } else if (k != MCR_KERNEL_VALU_CHUNK && n < 32 * kMfmaMaxT &&
+             (n >= kRegBelowN || k == MCR_KERNEL_VALU_TILE)) {
+    p->f32 = true;
+    p->T = (n + 1 + 31) / 32;
+    p->S = (n + 7) / 8;
   }
   return MCR_OK;
 }
@@ -426,6 +431,7 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   pa.n = q->n;
   pa.T = p.T;
   pa.S = p.S;
+  pa.f32 = p.f32;
   pa.info = st->d.info;
   pa.v64 = st->d.v64;
   pa.colpack = st->d.colpack;

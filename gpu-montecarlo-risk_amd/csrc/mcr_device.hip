@@ -21,6 +21,7 @@
 // normal ever leaves the chip.
 #include <map>
 #include <mutex>
+#include <tuple>
 
 #include "mcr_kern_common.h"
 
@@ -365,27 +366,33 @@ __device__ void prep_body(const PrepArgs& a, size_t gid, size_t gsz) {
       a.L32[l32_offset(r8, i, j)] = (i < n && j <= i) ? (float)L[(size_t)i * n + j] : 0.0f;
     }
   }
-  // MFMA: augmented rows (assets, zero pads, loss row 32T-1 = -v), hi/lo bf16
+  // MFMA: augmented rows (assets, zero pads, loss row 32T-1: -v and -w^T mu in
+  // bf16 hi/lo parts; v and w^T mu in fp32, whose kernels negate the sum as the
+  // register kernel does)
   if (a.T > 0) {
     const int T = a.T, S = a.S;
     const float mp32 = (float)a.info->mp;
+    auto entry = [&](int row, int k) {
+      if (k >= n) return 0.0f;
+      if (row < n) return k <= row ? (float)L[(size_t)row * n + k] : 0.0f;
+      if (row == 32 * T - 1) return a.f32 ? (float)a.v64[k] : -(float)a.v64[k];
+      return 0.0f;
+    };
     for (size_t e = gid; e < (size_t)T * S * 64; e += gsz) {
       const int lane = (int)(e % 64);
       const int s = (int)((e / 64) % S);
       const int t = (int)(e / (64 * (size_t)S));
       const int row = 32 * t + (lane & 31);
+      if (a.f32) {
+        const int k0 = 8 * s + (lane >> 5);
+        reinterpret_cast<float4*>(a.lfrag)[e] =
+            make_float4(entry(row, k0), entry(row, k0 + 2), entry(row, k0 + 4), entry(row, k0 + 6));
+        continue;
+      }
       const int k0 = 16 * s + 8 * (lane >> 5);
       uint16_t hb[8], lb[8];
       for (int q = 0; q < 8; ++q) {
-        const int k = k0 + q;
-        float m = 0.0f;
-        if (k < n) {
-          if (row < n) {
-            m = (k <= row) ? (float)L[(size_t)row * n + k] : 0.0f;
-          } else if (row == 32 * T - 1) {
-            m = -(float)a.v64[k];
-          }
-        }
+        const float m = entry(row, k0 + q);
         hb[q] = bf16_bits(m);
         lb[q] = bf16_bits(m - bf16_val(hb[q]));
       }
@@ -403,7 +410,8 @@ __device__ void prep_body(const PrepArgs& a, size_t gid, size_t gsz) {
     }
     for (size_t e = gid; e < (size_t)32 * T; e += gsz) {
       const int row = (int)e;
-      a.rowinit[e] = row < n ? (float)a.mu[row] : (row == 32 * T - 1 ? -mp32 : INFINITY);
+      a.rowinit[e] =
+          row < n ? (float)a.mu[row] : (row == 32 * T - 1 ? (a.f32 ? mp32 : -mp32) : INFINITY);
     }
   }
 }
@@ -770,24 +778,39 @@ hipError_t launch_normals(uint64_t seed, uint64_t path0, uint64_t npaths, int n,
 // ---------------------------------------------------------------------------
 static uint64_t min_u64(uint64_t x, uint64_t y) { return x < y ? x : y; }
 
-int resident_blocks(const void* kernel, int block) {
+int resident_blocks(const void* kernel, int block, size_t lds) {
   static std::mutex mu;
-  static std::map<std::pair<const void*, int>, int> cache;
+  static std::map<std::tuple<const void*, int, size_t>, int> cache;
   std::lock_guard<std::mutex> lk(mu);
-  auto it = cache.find({kernel, block});
+  auto it = cache.find({kernel, block, lds});
   if (it != cache.end()) return it->second;
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds) != hipSuccess ||
       per_cu < 1) {
     (void)hipGetLastError();
     per_cu = 1;
   }
-  cache[{kernel, block}] = per_cu;
+  cache[{kernel, block, lds}] = per_cu;
   return per_cu;
 }
 
 hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t stream) {
   if (a.npaths == 0) return hipSuccess;
+  if (kernel == 3) {
+    PathKernel k = mfma_kernel(a.n, a.T);
+    if (!k) return hipErrorInvalidValue;
+    const uint64_t blocks = min_u64((a.npaths + 255) / 256, (uint64_t)num_cus * 8);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    return hipGetLastError();
+  }
+  if (a.T > 0 && a.T <= kMfmaMaxT && kernel != 4) {
+    PathKernel k = wave_kernel(a.T);
+    const size_t lds = wave_lds(a.T, a.S);
+    const uint64_t per_cu = (uint64_t)resident_blocks((const void*)k, 256, lds);
+    const uint64_t blocks = min_u64((a.npaths + 255) / 256, (uint64_t)num_cus * per_cu);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), lds, stream, a);
+    return hipGetLastError();
+  }
   if (kernel == 1) {
     PathKernel k = reg_kernel(a.n);
     if (!k) return hipErrorInvalidValue;
@@ -838,13 +861,6 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
     const uint64_t per_cu = (uint64_t)resident_blocks((const void*)k, block);
     const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * per_cu);
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(block), 0, stream, a);
-    return hipGetLastError();
-  }
-  if (kernel == 3) {
-    PathKernel k = mfma_kernel(a.n, a.T);
-    if (!k) return hipErrorInvalidValue;
-    const uint64_t blocks = min_u64((a.npaths + 255) / 256, (uint64_t)num_cus * 8);
-    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, stream, a);
     return hipGetLastError();
   }
   return hipErrorInvalidValue;

@@ -16,6 +16,14 @@ constexpr int kBatchMaxN = kMfmaLdsMaxN;   // batches and the serving loop
 constexpr int kRegMaxN = 64;    // register kernel: one row accumulator per asset
 constexpr int kMfmaMaxT = 4;    // MFMA kernel: 32-row tiles (assets + loss row)
 constexpr int kMfmaNB = 32;     // MFMA kernel: Philox blocks per path (n <= 127)
+// fp32 queries below this run the register kernel, from it up to n = 127 the
+// wave kernel.  Per 64 paths the register kernel's n^2 / 2 multiply-adds read a
+// scalar operand and issue at half rate, the wave kernel's products take the
+// padded tiles' time: they meet at n = 62-63 (5.67 / 5.66 ms for 4e11 / (n^2 + 40
+// n) paths) and the third tile of n = 64 puts the wave kernel back (7.52 against
+// 5.85 ms); the register kernel is not built past 64, where the wave kernel takes
+// 6.1 ms (n = 80) and 4.6 ms (n = 127) against 8.8 ms of the tile kernel.
+constexpr int kRegBelowN = 65;
 
 constexpr int kTilePaths = 64;  // paths per workgroup in the tile kernel
 constexpr int kTileRows = 8;    // rows per register block in the tile kernel
@@ -69,9 +77,10 @@ struct PathArgs {
   const float* L32;      // tile kernel: fp32 factor in 8 x 4 blocks (l32_offset)
   const float* mu32;     // [n]
   const float* v32;      // [n] L^T w
-  const uint4* lfrag;    // MFMA: [T][S][64 lanes][hi, lo] 8 x bf16 each
+  const uint4* lfrag;    // MFMA: [T][S][64 lanes][hi, lo] 8 x bf16 each, or fp32
+                         // [T][S][64 lanes] float4
   const float* rowinit;  // MFMA: [32 T] row initial values
-  int T, S;              // MFMA tiles and 16-wide K steps
+  int T, S;              // MFMA tiles and 16-wide K steps (fp32: 8-wide octets)
   const DevInfo* info;
   DevAccum* acc;
   int32_t* S_out;        // optional [npaths]
@@ -109,6 +118,7 @@ struct PrepArgs {
   const double* L;   // [n*n]
   const double* mu;  // [n]
   int n, T, S;
+  int f32;           // lfrag holds fp32 fragments (S octets), else bf16 hi/lo
   const DevInfo* info;
   double* v64;       // [n] scratch: L^T w
   float* colpack;
@@ -154,10 +164,12 @@ int big_range(int T);                          // range of T (T >= 5)
 int batch_big_shapes(int range);               // shapes of a range
 BatchKernel batch_big_kernel(int T, int shape);  // T <= 24, 64 * batch_big_waves threads
 int batch_big_waves(int T, int shape);         // waves per workgroup of that kernel
-int resident_blocks(const void* kernel, int block);  // workgroups per CU (occupancy)
+// workgroups per CU (occupancy) with lds bytes of dynamic LDS
+int resident_blocks(const void* kernel, int block, size_t lds = 0);
 hipError_t launch_batch_clear(unsigned* next, int count, hipStream_t stream);
 hipError_t launch_batch_kernel(BatchKernel k, const BatchArgs& b, int grid, int block,
                                hipStream_t stream);
+size_t wave_lds(int T, int S);  // dynamic LDS of the fp32 wave kernel
 hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t stream);
 hipError_t launch_normals(uint64_t seed, uint64_t path0, uint64_t npaths, int n, float* out,
                           hipStream_t stream);

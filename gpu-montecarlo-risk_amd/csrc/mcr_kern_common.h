@@ -318,6 +318,7 @@ __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t w[4]) {
 
 typedef void (*PathKernel)(PathArgs);
 PathKernel reg_kernel(int n);          // mcr_reg.hip
+PathKernel wave_kernel(int T);         // mcr_wave.hip
 PathKernel mfma_kernel(int n, int T);  // mcr_mfma.hip
 PathKernel mfma_big_kernel(int T);     // mcr_mfma_big.hip
 

@@ -131,6 +131,15 @@ def test_tile_kernel_exact(mcr, orc, n):
     assert r.kernel == "valu_tile"
 
 
+@pytest.mark.parametrize("n", [31, 32, 62, 63, 64, 90, 95, 96, 97, 126, 127])
+def test_wave_kernel_exact(mcr, orc, n):
+    """The fp32 wave kernel at the edges of its 32-row tiles, 8-column octets
+    and half blocks, over paths whose ids cross 2^32 inside a 64-path group."""
+    r = _exact_case(mcr, orc, n, 5000, max(1, n // 5), mcr.KERNEL_VALU_TILE,
+                    path_offset=2**32 - 2469)
+    assert r.kernel == "valu_tile"
+
+
 @pytest.mark.parametrize("n", [1, 5, 9, 50, 129, 257, 600, 608, 609, 700, 1000, 1024])
 def test_chunk_kernel_exact(mcr, orc, n):
     """The column-chunk kernel (any n <= 1024; fp32 past 608): per-path
