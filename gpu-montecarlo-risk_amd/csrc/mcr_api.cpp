@@ -175,7 +175,7 @@ struct DevBuffers {
   double *A, *mu, *w, *L, *v64;
   DevInfo* info;
   DevAccum* acc;
-  float *colpack, *L32, *mu32, *v32, *rowinit;
+  float *colpack, *mu32, *v32, *rowinit;
   uint4* lfrag;
   float* gather;
   unsigned* hist;
@@ -185,8 +185,8 @@ struct DevBuffers {
 };
 
 struct Plan {
-  int n, T, S, r8;
-  bool f32;  // fp32 fragments (S octets) in lfrag
+  int n, T, S;
+  F32Form f32;  // fp32 fragments (S octets) in lfrag
   int kernel;
   int n_alpha;
   bool per_path;
@@ -203,8 +203,7 @@ size_t layout(const Plan& p, char* base, DevBuffers* b) {
   b->v64 = c.take<double>(n);
   b->info = c.take<DevInfo>(1);
   b->acc = c.take<DevAccum>(1);
-  b->colpack = c.take<float>(colpack_size(p.n));
-  b->L32 = c.take<float>((size_t)p.r8 * p.r8);
+  b->colpack = p.T ? nullptr : c.take<float>(colpack_size(p.n));  // register kernel
   b->mu32 = c.take<float>(n);
   b->v32 = c.take<float>(n);
   b->lfrag = c.take<uint4>((size_t)p.T * p.S * 64 * (p.f32 ? 1 : 2));
@@ -271,14 +270,17 @@ int choose_kernel(const mcr_query* q, Plan* p) {
   }
   p->kernel = k;
   p->T = p->S = 0;
-  p->f32 = false;
+  p->f32 = kF32None;
   if (k == MCR_KERNEL_MFMA || k == MCR_KERNEL_MFMA_LDS) {
     p->T = (n + 1 + 31) / 32;
     p->S = (n + 15) / 16;
-  } else if (k != MCR_KERNEL_VALU_CHUNK && n < 32 * kMfmaMaxT &&
-             (n >= kRegBelowN || k == MCR_KERNEL_VALU_TILE)) {
-    p->f32 = true;
+  } else if (k == MCR_KERNEL_VALU_TILE && n < 32 * kMfmaMaxT) {
+    p->f32 = kF32Wave;
     p->T = (n + 1 + 31) / 32;
+    p->S = (n + 7) / 8;
+  } else if (k != MCR_KERNEL_VALU_REG) {
+    p->f32 = kF32Lds;
+    p->T = (n + 31) / 32;
     p->S = (n + 7) / 8;
   }
   return MCR_OK;
@@ -345,7 +347,6 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   Plan& p = st->plan;
   p.n = q->n;
   MCR_TRY(choose_kernel(q, &p));
-  p.r8 = ((q->n + kTileRows - 1) / kTileRows) * kTileRows;
   p.n_alpha = (q->flags & MCR_F_VAR) ? q->n_alpha : 0;
   p.per_path = q->S_out || q->loss_out;
   p.chunk = p.per_path ? (size_t)std::min<uint64_t>((uint64_t)q->paths,
@@ -435,7 +436,6 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   pa.info = st->d.info;
   pa.v64 = st->d.v64;
   pa.colpack = st->d.colpack;
-  pa.L32 = st->d.L32;
   pa.mu32 = st->d.mu32;
   pa.v32 = st->d.v32;
   pa.lfrag = st->d.lfrag;
@@ -489,13 +489,13 @@ PathArgs base_args(const mcr_query* q, const Staged& st) {
     a.thr_hi = 0.0f;  // lo > hi: near accounting off
   }
   a.colpack = st.d.colpack;
-  a.L32 = st.d.L32;
   a.mu32 = st.d.mu32;
   a.v32 = st.d.v32;
   a.lfrag = st.d.lfrag;
   a.rowinit = st.d.rowinit;
   a.T = st.plan.T;
   a.S = st.plan.S;
+  a.f32 = st.plan.f32;
   a.info = st.d.info;
   a.acc = st.d.acc;
   a.gather = st.d.gather;
@@ -1536,10 +1536,10 @@ int mcr_prepare(const mcr_query* q, mcr_model_export* out) {
   if (out->L64)
     HIP_TRY(hipMemcpy(out->L64, st.d.L, (size_t)n * n * sizeof(double), hipMemcpyDeviceToHost));
   if (out->L32) {
-    std::vector<float> l((size_t)st.plan.r8 * st.plan.r8);
-    HIP_TRY(hipMemcpy(l.data(), st.d.L32, l.size() * sizeof(float), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j) out->L32[(size_t)i * n + j] = l[l32_offset(st.plan.r8, i, j)];
+    // every layout rounds the FP64 factor's entries, to nearest
+    std::vector<double> l((size_t)n * n);
+    HIP_TRY(hipMemcpy(l.data(), st.d.L, l.size() * sizeof(double), hipMemcpyDeviceToHost));
+    for (size_t e = 0; e < l.size(); ++e) out->L32[e] = (float)l[e];
   }
   if (out->mu32) HIP_TRY(hipMemcpy(out->mu32, st.d.mu32, n * sizeof(float), hipMemcpyDeviceToHost));
   if (out->v32) HIP_TRY(hipMemcpy(out->v32, st.d.v32, n * sizeof(float), hipMemcpyDeviceToHost));

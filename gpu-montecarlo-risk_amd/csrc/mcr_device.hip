@@ -11,8 +11,10 @@
 //   k_valu_reg   fused path kernel, one path per lane, n <= 64 rows in registers,
 //                factor read through the scalar cache: r_i = mu_i then fmaf(L_ij, z_j)
 //                for j = 0..i, exactly the order the C mirror uses.
-//   k_valu_tile  fused path kernel for n <= 608: 64 paths per workgroup, their
-//                normals staged once in LDS, rows in 8-row register blocks.
+//   k_wave       fp32, 64 < n <= 127: 64 paths per wave on v_mfma_f32_32x32x2_f32,
+//                whose row sums are the same fmaf chains.
+//   k_f32_lds    fp32, n <= 1024: 64 paths per workgroup, their normals staged in
+//                LDS as operands of the same instruction.
 //   k_mfma       32 paths per wave on v_mfma_f32_32x32x16_bf16: A = factor rows
 //                (bf16 hi/lo), B = normals (bf16 hi/lo), three products per step
 //                (hi*hi + hi*lo + lo*hi), fp32 accumulation, n <= 127.
@@ -342,40 +344,38 @@ hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStre
 }
 
 // ---------------------------------------------------------------------------
-// Prep: layouts of the factor for the three path kernels.
+// Prep: layouts of the factor for the path kernels.
 // ---------------------------------------------------------------------------
 __device__ void prep_body(const PrepArgs& a, size_t gid, size_t gsz) {
   const int n = a.n;
   const double* __restrict__ L = a.L;
-  const int r8 = ((n + kTileRows - 1) / kTileRows) * kTileRows;
-  if (a.colpack) {
-    // fp32 loading and mean
+  if (a.v32) {
     for (size_t e = gid; e < (size_t)n; e += gsz) {
       a.v32[e] = (float)a.v64[e];
       a.mu32[e] = (float)a.mu[e];
-      a.colpack[colpack_offset(n, (int)e) + n - (int)e] = (float)a.v64[e];
     }
-    // register kernel: column-packed lower triangle
+  }
+  if (a.colpack) {
+    // register kernel: column-packed lower triangle and loading
+    for (size_t e = gid; e < (size_t)n; e += gsz)
+      a.colpack[colpack_offset(n, (int)e) + n - (int)e] = (float)a.v64[e];
     for (size_t e = gid; e < (size_t)n * n; e += gsz) {
       const int i = (int)(e / n), j = (int)(e % n);
       if (j <= i) a.colpack[colpack_offset(n, j) + i - j] = (float)L[e];
     }
-    // tile kernel: zero-padded r8 x r8 in 8 x 4 blocks (l32_offset)
-    for (size_t e = gid; e < (size_t)r8 * r8; e += gsz) {
-      const int i = (int)(e / r8), j = (int)(e % r8);
-      a.L32[l32_offset(r8, i, j)] = (i < n && j <= i) ? (float)L[(size_t)i * n + j] : 0.0f;
-    }
   }
   // MFMA: augmented rows (assets, zero pads, loss row 32T-1: -v and -w^T mu in
-  // bf16 hi/lo parts; v and w^T mu in fp32, whose kernels negate the sum as the
-  // register kernel does)
+  // bf16 hi/lo parts; v and w^T mu in the fp32 wave kernel's, which negates the
+  // sum as the register kernel does; likewise in the fp32 LDS kernel's unless
+  // its tiles have no row to spare: row < n comes first)
   if (a.T > 0) {
     const int T = a.T, S = a.S;
     const float mp32 = (float)a.info->mp;
     auto entry = [&](int row, int k) {
       if (k >= n) return 0.0f;
       if (row < n) return k <= row ? (float)L[(size_t)row * n + k] : 0.0f;
-      if (row == 32 * T - 1) return a.f32 ? (float)a.v64[k] : -(float)a.v64[k];
+      if (row == 32 * T - 1)
+        return a.f32 ? (float)a.v64[k] : -(float)a.v64[k];
       return 0.0f;
     };
     for (size_t e = gid; e < (size_t)T * S * 64; e += gsz) {
@@ -411,7 +411,8 @@ __device__ void prep_body(const PrepArgs& a, size_t gid, size_t gsz) {
     for (size_t e = gid; e < (size_t)32 * T; e += gsz) {
       const int row = (int)e;
       a.rowinit[e] =
-          row < n ? (float)a.mu[row] : (row == 32 * T - 1 ? (a.f32 ? mp32 : -mp32) : INFINITY);
+          row < n ? (float)a.mu[row]
+                  : (row == 32 * T - 1 ? (a.f32 ? mp32 : -mp32) : INFINITY);
     }
   }
 }
@@ -435,318 +436,12 @@ hipError_t launch_prep_batch(const PrepArgs* pas, int nq, int max_n, hipStream_t
 }
 
 hipError_t launch_prep(const PrepArgs& a, hipStream_t stream) {
-  size_t work = (size_t)a.n * a.n;
-  const int r8 = ((a.n + kTileRows - 1) / kTileRows) * kTileRows;
-  if ((size_t)r8 * r8 > work) work = (size_t)r8 * r8;
+  const size_t work = (size_t)a.n * a.n;
   int blocks = (int)((work + 255) / 256);
   if (blocks > 1024) blocks = 1024;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(k_prep, dim3(blocks), dim3(256), 0, stream, a);
   return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Tile kernel: 64 paths per workgroup (lane = path), NW waves.  Phase 1 writes
-// the paths' normals to LDS as float4 [block][lane]; phase 2 splits the rows
-// into 8-row register blocks dealt to the waves in snake order (block cost grows
-// with the row index), the loss row being one more block.  Row i still sees
-// mu_i, then z_0 .. z_i in order, so results equal the register kernel's.
-// The normals of 64 paths take up to 152 KiB, so at large n one workgroup
-// fills a CU's LDS: NW grows as fewer workgroups fit (4, 8, 16 waves), keeping
-// several waves per SIMD to cover the scalar factor loads and LDS reads.
-// ---------------------------------------------------------------------------
-constexpr int kTileStaticLds = 16 * 64 * 4 + 64 * 4 + (kMaxN + 1) * 4;
-
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_valu_tile(PathArgs a) {
-  extern __shared__ float4 zs[];  // [nb][64]
-  __shared__ int sS[NW][64];
-  __shared__ float sLoss[64];
-  __shared__ unsigned sh_hist[kMaxN + 1];
-  const int n = a.n;
-  const int nb = (n + 3) >> 2;
-  const int nrb = (n + kTileRows - 1) / kTileRows;
-  const int ldl = nrb * kTileRows;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool want_hist = a.s_hist != nullptr;
-  if (want_hist) {
-    for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
-  }
-  MCR_CONSTP(float) L = cview(a.L32);
-  MCR_CONSTP(float) mu = cview(a.mu32);
-  MCR_CONSTP(float) v = cview(a.v32);
-  const float mp32 = (float)cview(a.info)->mp;
-  const Key2 key = key_of(a.seed);
-  const bool want_near = a.thr_lo < a.thr_hi;
-  LaneTally t;
-  zero_tally(t);
-
-  for (uint64_t tile = blockIdx.x; tile * kTilePaths < a.npaths; tile += gridDim.x) {
-    const uint64_t q = tile * kTilePaths + lane;
-    const uint64_t path = a.path0 + q;
-    for (int b = wave; b < nb; b += NW) {
-      float z[4];
-      normals4(key, path, (uint32_t)b, z);
-      zs[b * 64 + lane] = make_float4(z[0], z[1], z[2], z[3]);
-    }
-    __syncthreads();
-
-    int S = 0;
-    bool near = false;
-    for (int rb = 0; rb <= nrb; ++rb) {
-      const int p = rb / NW, rw = rb % NW;
-      const int owner = (p & 1) ? NW - 1 - rw : rw;
-      if (owner != wave) continue;
-      if (rb == nrb) {
-        // loss row: g = w^T mu + sum_j v_j z_j, j ascending
-        float g = mp32;
-        for (int jb = 0; jb < nb - 1; ++jb) {
-          const float4 z4 = zs[jb * 64 + lane];
-          g = __builtin_fmaf(v[4 * jb + 0], z4.x, g);
-          g = __builtin_fmaf(v[4 * jb + 1], z4.y, g);
-          g = __builtin_fmaf(v[4 * jb + 2], z4.z, g);
-          g = __builtin_fmaf(v[4 * jb + 3], z4.w, g);
-        }
-        {
-          const int jb = nb - 1;
-          const float4 z4 = zs[jb * 64 + lane];
-          const int rem = n - 4 * jb;
-          g = __builtin_fmaf(v[4 * jb + 0], z4.x, g);
-          if (rem > 1) g = __builtin_fmaf(v[4 * jb + 1], z4.y, g);
-          if (rem > 2) g = __builtin_fmaf(v[4 * jb + 2], z4.z, g);
-          if (rem > 3) g = __builtin_fmaf(v[4 * jb + 3], z4.w, g);
-        }
-        sLoss[lane] = -g;
-        continue;
-      }
-      const int i0 = rb * kTileRows;
-      float acc[kTileRows];
-#pragma unroll
-      for (int r = 0; r < kTileRows; ++r) acc[r] = (i0 + r < n) ? mu[i0 + r] : 0.0f;
-      // Row block rb's 8 x 4 factor blocks (32 floats each, column block jb at
-      // Lb + 32 jb): one K step is two 64-byte scalar loads.
-      MCR_CONSTP(float) Lb = L + l32_offset(ldl, i0, 0);
-      const int J = i0 / 4;
-      // Two K steps per wait where the row blocks are long (NW >= 8: n >~ 150;
-      // n = 400 -8 %); with four waves the unrolled loop measured slower.
-      constexpr int kStepUnroll = NW >= 8 ? 2 : 1;
-#pragma unroll kStepUnroll
-      for (int jb = 0; jb < J; ++jb) {
-        const float4 z4 = zs[jb * 64 + lane];
-        MCR_CONSTP(float) lv = Lb + 32 * jb;
-#pragma unroll
-        for (int r = 0; r < kTileRows; ++r) {
-          acc[r] = __builtin_fmaf(lv[4 * r + 0], z4.x, acc[r]);
-          acc[r] = __builtin_fmaf(lv[4 * r + 1], z4.y, acc[r]);
-          acc[r] = __builtin_fmaf(lv[4 * r + 2], z4.z, acc[r]);
-          acc[r] = __builtin_fmaf(lv[4 * r + 3], z4.w, acc[r]);
-        }
-      }
-      // diagonal 8x8 block: row i0+r uses columns i0 .. i0+r
-      float zd[8];
-      {
-        const float4 z4 = zs[(i0 / 4) * 64 + lane];
-        zd[0] = z4.x; zd[1] = z4.y; zd[2] = z4.z; zd[3] = z4.w;
-        if (i0 / 4 + 1 < nb) {
-          const float4 z5 = zs[(i0 / 4 + 1) * 64 + lane];
-          zd[4] = z5.x; zd[5] = z5.y; zd[6] = z5.z; zd[7] = z5.w;
-        } else {
-          zd[4] = zd[5] = zd[6] = zd[7] = 0.0f;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < kTileRows; ++r) {
-#pragma unroll
-        for (int c = 0; c <= r; ++c)
-          acc[r] = __builtin_fmaf(Lb[32 * (J + (c >> 2)) + 4 * r + (c & 3)], zd[c], acc[r]);
-      }
-#pragma unroll
-      for (int r = 0; r < kTileRows; ++r) {
-        if (i0 + r < n) {
-          S += (acc[r] < a.thr) ? 1 : 0;
-          if (want_near) near |= (acc[r] >= a.thr_lo) & (acc[r] <= a.thr_hi);
-        }
-      }
-    }
-    sS[wave][lane] = S | (near ? (1 << 30) : 0);
-    __syncthreads();
-    if (wave == 0 && q < a.npaths) {
-      int tot = 0;
-      bool nr = false;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const int e = sS[w][lane];
-        tot += e & 0xffff;
-        nr |= (e >> 30) & 1;
-      }
-      tally_path(a, t, q, tot, sLoss[lane], nr, want_hist ? sh_hist : nullptr);
-    }
-    __syncthreads();
-  }
-  flush_tally(a, t);
-  if (want_hist) {
-    __syncthreads();
-    for (int i = threadIdx.x; i <= n; i += blockDim.x)
-      if (sh_hist[i]) atomicAdd(&a.s_hist[i], (unsigned long long)sh_hist[i]);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Column-chunk kernel for n up to kChunkMaxN (and any smaller n): 64 paths per
-// workgroup, 16 waves.  The paths' normals no longer fit the LDS whole, so the
-// columns are taken in chunks of kChunkBlocks 4-column blocks (512 columns,
-// 128 KiB): the waves generate a chunk's normals into LDS, then every wave
-// advances all of its 8-row register blocks (snake order, the loss row one
-// more block) over the chunk's columns.  Each wave's blocks stay in registers
-// across the chunks, so row i still sees mu_i, then z_0 .. z_i in order and
-// the results equal the tile and register kernels' bit for bit.
-// ---------------------------------------------------------------------------
-constexpr int kChunkBlocks = 128;  // 4-column blocks per chunk (even: a diagonal
-                                   // block's two column blocks share a chunk)
-constexpr int kChunkNW = 16;
-constexpr int kChunkMB = (kChunkMaxN / kTileRows + kChunkNW - 1) / kChunkNW;  // row blocks per wave
-
-__global__ __launch_bounds__(64 * kChunkNW) void k_valu_chunk(PathArgs a) {
-  constexpr int NW = kChunkNW;
-  __shared__ float4 zs[kChunkBlocks * 64];  // [block - chunk start][lane]
-  __shared__ int sS[NW][64];
-  __shared__ float sLoss[64];
-  __shared__ unsigned sh_hist[kChunkMaxN + 1];
-  const int n = a.n;
-  const int nb = (n + 3) >> 2;
-  const int nrb = (n + kTileRows - 1) / kTileRows;  // row blocks
-  const int ldl = nrb * kTileRows;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // the loss row goes to the wave the snake deal would give block nrb
-  const bool loss_wave = ((nrb / NW) & 1 ? NW - 1 - nrb % NW : nrb % NW) == wave;
-  const bool want_hist = a.s_hist != nullptr;
-  if (want_hist) {
-    for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
-  }
-  MCR_CONSTP(float) L = cview(a.L32);
-  MCR_CONSTP(float) mu = cview(a.mu32);
-  MCR_CONSTP(float) v = cview(a.v32);
-  const float mp32 = (float)cview(a.info)->mp;
-  const Key2 key = key_of(a.seed);
-  const bool want_near = a.thr_lo < a.thr_hi;
-  LaneTally t;
-  zero_tally(t);
-
-  for (uint64_t tile = blockIdx.x; tile * kTilePaths < a.npaths; tile += gridDim.x) {
-    const uint64_t q = tile * kTilePaths + lane;
-    const uint64_t path = a.path0 + q;
-    // this wave's k-th row block: rb = k NW + (k odd ? NW - 1 - wave : wave)
-    float acc[kChunkMB][kTileRows];
-#pragma unroll
-    for (int k = 0; k < kChunkMB; ++k) {
-      const int rb = k * NW + ((k & 1) ? NW - 1 - wave : wave);
-#pragma unroll
-      for (int r = 0; r < kTileRows; ++r) {
-        const int i = rb * kTileRows + r;
-        acc[k][r] = (rb < nrb && i < n) ? mu[i] : 0.0f;
-      }
-    }
-    float g = mp32;  // loss row: g = w^T mu + sum_j v_j z_j, j ascending
-    for (int jb0 = 0; jb0 < nb; jb0 += kChunkBlocks) {
-      const int jb1 = min(nb, jb0 + kChunkBlocks);
-      // a fresh copy of the wave index per chunk keeps the compiler from
-      // holding every block's addresses across the chunk loop (SGPR spills)
-      int wv = wave;
-      asm volatile("" : "+s"(wv));
-      for (int b = jb0 + wv; b < jb1; b += NW) {
-        float z[4];
-        normals4(key, path, (uint32_t)b, z);
-        zs[(b - jb0) * 64 + lane] = make_float4(z[0], z[1], z[2], z[3]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int k = 0; k < kChunkMB; ++k) {
-        const int rb = k * NW + ((k & 1) ? NW - 1 - wv : wv);
-        if (rb >= nrb) continue;
-        const int i0 = rb * kTileRows;
-        const int J = i0 / 4;  // column blocks left of the diagonal block
-        MCR_CONSTP(float) Lb = L + l32_offset(ldl, i0, 0);
-        const int je = min(jb1, J);
-        for (int jb = jb0; jb < je; ++jb) {
-          const float4 z4 = zs[(jb - jb0) * 64 + lane];
-          MCR_CONSTP(float) lv = Lb + 32 * jb;
-#pragma unroll
-          for (int r = 0; r < kTileRows; ++r) {
-            acc[k][r] = __builtin_fmaf(lv[4 * r + 0], z4.x, acc[k][r]);
-            acc[k][r] = __builtin_fmaf(lv[4 * r + 1], z4.y, acc[k][r]);
-            acc[k][r] = __builtin_fmaf(lv[4 * r + 2], z4.z, acc[k][r]);
-            acc[k][r] = __builtin_fmaf(lv[4 * r + 3], z4.w, acc[k][r]);
-          }
-        }
-        if (J >= jb0 && J < jb1) {
-          // diagonal 8x8 block (column blocks J and J+1, both in this chunk)
-          float zd[8];
-          const float4 z4 = zs[(J - jb0) * 64 + lane];
-          zd[0] = z4.x; zd[1] = z4.y; zd[2] = z4.z; zd[3] = z4.w;
-          if (J + 1 < nb) {
-            const float4 z5 = zs[(J + 1 - jb0) * 64 + lane];
-            zd[4] = z5.x; zd[5] = z5.y; zd[6] = z5.z; zd[7] = z5.w;
-          } else {
-            zd[4] = zd[5] = zd[6] = zd[7] = 0.0f;
-          }
-#pragma unroll
-          for (int r = 0; r < kTileRows; ++r) {
-#pragma unroll
-            for (int c = 0; c <= r; ++c)
-              acc[k][r] = __builtin_fmaf(Lb[32 * (J + (c >> 2)) + 4 * r + (c & 3)], zd[c], acc[k][r]);
-          }
-        }
-      }
-      if (loss_wave) {
-        for (int jb = jb0; jb < jb1; ++jb) {
-          const float4 z4 = zs[(jb - jb0) * 64 + lane];
-          const int rem = n - 4 * jb;  // >= 4 except in the last block
-          g = __builtin_fmaf(v[4 * jb + 0], z4.x, g);
-          if (rem > 1) g = __builtin_fmaf(v[4 * jb + 1], z4.y, g);
-          if (rem > 2) g = __builtin_fmaf(v[4 * jb + 2], z4.z, g);
-          if (rem > 3) g = __builtin_fmaf(v[4 * jb + 3], z4.w, g);
-        }
-      }
-      __syncthreads();  // the chunk's normals are read; the next chunk may overwrite them
-    }
-
-    if (loss_wave) sLoss[lane] = -g;
-    int S = 0;
-    bool near = false;
-#pragma unroll
-    for (int k = 0; k < kChunkMB; ++k) {
-      const int rb = k * NW + ((k & 1) ? NW - 1 - wave : wave);
-      if (rb >= nrb) continue;
-#pragma unroll
-      for (int r = 0; r < kTileRows; ++r) {
-        if (rb * kTileRows + r < n) {
-          S += (acc[k][r] < a.thr) ? 1 : 0;
-          if (want_near) near |= (acc[k][r] >= a.thr_lo) & (acc[k][r] <= a.thr_hi);
-        }
-      }
-    }
-    sS[wave][lane] = S | (near ? (1 << 30) : 0);
-    __syncthreads();
-    if (wave == 0 && q < a.npaths) {
-      int tot = 0;
-      bool nr = false;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const int e = sS[w][lane];
-        tot += e & 0xffff;
-        nr |= (e >> 30) & 1;
-      }
-      tally_path(a, t, q, tot, sLoss[lane], nr, want_hist ? sh_hist : nullptr);
-    }
-    __syncthreads();
-  }
-  flush_tally(a, t);
-  if (want_hist) {
-    __syncthreads();
-    for (int i = threadIdx.x; i <= n; i += blockDim.x)
-      if (sh_hist[i]) atomicAdd(&a.s_hist[i], (unsigned long long)sh_hist[i]);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -803,7 +498,7 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, stream, a);
     return hipGetLastError();
   }
-  if (a.T > 0 && a.T <= kMfmaMaxT && kernel != 4) {
+  if (a.f32 == kF32Wave) {
     PathKernel k = wave_kernel(a.T);
     const size_t lds = wave_lds(a.T, a.S);
     const uint64_t per_cu = (uint64_t)resident_blocks((const void*)k, 256, lds);
@@ -811,47 +506,29 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), lds, stream, a);
     return hipGetLastError();
   }
+  if (a.f32 == kF32Lds) {
+    if (a.n < 1 || a.n > kChunkMaxN) return hipErrorInvalidValue;
+    const F32Shape s = f32_shape(a.n);
+    static bool attr = false;
+    if (!attr) {
+      // the largest dynamic request; static LDS comes on top (160 KiB in all)
+      const int max_dyn = (int)f32_shape(kMaxN).lds;
+      for (int n : {kMaxN, 256, 128}) {
+        const hipError_t e = hipFuncSetAttribute((const void*)f32_shape(n).kernel,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, max_dyn);
+        if (e != hipSuccess) return e;
+      }
+      attr = true;
+    }
+    const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * s.per_cu);
+    hipLaunchKernelGGL(s.kernel, dim3((unsigned)blocks), dim3(64 * s.waves), s.lds, stream, a);
+    return hipGetLastError();
+  }
   if (kernel == 1) {
     PathKernel k = reg_kernel(a.n);
     if (!k) return hipErrorInvalidValue;
     const uint64_t blocks = min_u64((a.npaths + 255) / 256, (uint64_t)num_cus * 8);
     hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, stream, a);
-    return hipGetLastError();
-  }
-  if (kernel == 2) {
-    if (a.n < 1 || a.n > kMaxN) return hipErrorInvalidValue;
-    const int nb = (a.n + 3) >> 2;
-    const size_t lds = (size_t)nb * 64 * sizeof(float4);
-    static bool attr = false;
-    if (!attr) {
-      // the largest dynamic request (n = kMaxN); static LDS comes on top
-      const int max_dyn = ((kMaxN + 3) / 4) * 64 * (int)sizeof(float4);
-      for (const void* f : {(const void*)k_valu_tile<4>, (const void*)k_valu_tile<8>,
-                            (const void*)k_valu_tile<16>}) {
-        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_dyn);
-        if (e != hipSuccess) return e;
-      }
-      attr = true;
-    }
-    uint64_t per_cu = (160 * 1024) / (lds + kTileStaticLds);
-    if (per_cu < 1) per_cu = 1;
-    if (per_cu > 8) per_cu = 8;
-    const uint64_t blocks = min_u64((a.npaths + kTilePaths - 1) / kTilePaths, (uint64_t)num_cus * per_cu);
-    // waves per workgroup: about 16 per CU where the LDS limits the
-    // workgroups, at most 8 per SIMD
-    if (per_cu == 1)
-      hipLaunchKernelGGL(k_valu_tile<16>, dim3((unsigned)blocks), dim3(1024), lds, stream, a);
-    else if (per_cu <= 3)
-      hipLaunchKernelGGL(k_valu_tile<8>, dim3((unsigned)blocks), dim3(512), lds, stream, a);
-    else
-      hipLaunchKernelGGL(k_valu_tile<4>, dim3((unsigned)blocks), dim3(256), lds, stream, a);
-    return hipGetLastError();
-  }
-  if (kernel == 5) {
-    if (a.n < 1 || a.n > kChunkMaxN) return hipErrorInvalidValue;
-    // one 1024-thread workgroup per CU (139.5 KiB of LDS)
-    const uint64_t blocks = min_u64((a.npaths + kTilePaths - 1) / kTilePaths, (uint64_t)num_cus);
-    hipLaunchKernelGGL(k_valu_chunk, dim3((unsigned)blocks), dim3(64 * kChunkNW), 0, stream, a);
     return hipGetLastError();
   }
   if (kernel == 4) {

@@ -8,29 +8,28 @@
 namespace mcr {
 
 constexpr int kMaxAlpha = 4;
-constexpr int kMaxN = 608;      // tile kernel: 64 paths x n normals in LDS (152 KiB)
-constexpr int kChunkMaxN = 1024;  // column-chunk kernel and the factor: one thread per row
+constexpr int kMaxN = 608;      // fp32 LDS kernel: 64 paths x n normals in LDS at once (152 KiB)
+constexpr int kChunkMaxN = 1024;  // in chunks of columns; the factor: one thread per row
 constexpr int kMfmaLdsMaxN = 32 * 24 - 1;  // LDS MFMA kernels: 24 row tiles of 32
                                            // (assets + loss row)
 constexpr int kBatchMaxN = kMfmaLdsMaxN;   // batches and the serving loop
-constexpr int kRegMaxN = 64;    // register kernel: one row accumulator per asset
+// Register kernel: one row accumulator per asset.  Its n^2 / 2 multiply-adds per
+// path read a scalar operand and issue at half rate, the wave kernel's products
+// take the padded tiles' time: they meet at n = 62-63 (5.67 / 5.66 ms for 4e11 /
+// (n^2 + 40 n) paths) and the third tile of n = 64 puts the wave kernel back (7.52
+// against 5.85 ms); past 64 the wave kernel takes 6.1 ms (n = 80) and 4.6 ms (n =
+// 127).
+constexpr int kRegMaxN = 64;
 constexpr int kMfmaMaxT = 4;    // MFMA kernel: 32-row tiles (assets + loss row)
 constexpr int kMfmaNB = 32;     // MFMA kernel: Philox blocks per path (n <= 127)
-// fp32 queries below this run the register kernel, from it up to n = 127 the
-// wave kernel.  Per 64 paths the register kernel's n^2 / 2 multiply-adds read a
-// scalar operand and issue at half rate, the wave kernel's products take the
-// padded tiles' time: they meet at n = 62-63 (5.67 / 5.66 ms for 4e11 / (n^2 + 40
-// n) paths) and the third tile of n = 64 puts the wave kernel back (7.52 against
-// 5.85 ms); the register kernel is not built past 64, where the wave kernel takes
-// 6.1 ms (n = 80) and 4.6 ms (n = 127) against 8.8 ms of the tile kernel.
-constexpr int kRegBelowN = 65;
 
-constexpr int kTilePaths = 64;  // paths per workgroup in the tile kernel
-constexpr int kTileRows = 8;    // rows per register block in the tile kernel
 constexpr unsigned kGatherCap = 1u << 18;  // loss values kept per VaR window
 constexpr unsigned kBatchGatherCap = 1u << 16;  // per window, per query of a batch
 constexpr int kHistBins = 4096;            // refinement histogram
 
+// fp32 matrix kernels: none (bf16 or register kernel), the wave kernel's form (loss
+// row 32T-1 among the rows) or the LDS kernel's (rows only).
+enum F32Form : int { kF32None = 0, kF32Wave = 1, kF32Lds = 2 };
 enum LossMode : int { kLossNone = 0, kLossBracket = 1, kLossHist = 2 };
 
 // Written on the device by the factor kernel, read by the path kernels and
@@ -74,13 +73,13 @@ struct PathArgs {
   float thr;        // (float)(-x)
   float thr_lo, thr_hi;  // thr -/+ 1 ulp (near-threshold accounting)
   const float* colpack;  // register kernel: column j = L[j..n-1][j], v[j]
-  const float* L32;      // tile kernel: fp32 factor in 8 x 4 blocks (l32_offset)
   const float* mu32;     // [n]
   const float* v32;      // [n] L^T w
   const uint4* lfrag;    // MFMA: [T][S][64 lanes][hi, lo] 8 x bf16 each, or fp32
                          // [T][S][64 lanes] float4
   const float* rowinit;  // MFMA: [32 T] row initial values
   int T, S;              // MFMA tiles and 16-wide K steps (fp32: 8-wide octets)
+  int f32;               // F32Form of the fragments
   const DevInfo* info;
   DevAccum* acc;
   int32_t* S_out;        // optional [npaths]
@@ -118,11 +117,10 @@ struct PrepArgs {
   const double* L;   // [n*n]
   const double* mu;  // [n]
   int n, T, S;
-  int f32;           // lfrag holds fp32 fragments (S octets), else bf16 hi/lo
+  int f32;           // F32Form: lfrag holds fp32 fragments (S octets), else bf16 hi/lo
   const DevInfo* info;
   double* v64;       // [n] scratch: L^T w
   float* colpack;
-  float* L32;
   float* mu32;
   float* v32;
   uint4* lfrag;
@@ -175,13 +173,6 @@ hipError_t launch_normals(uint64_t seed, uint64_t path0, uint64_t npaths, int n,
                           hipStream_t stream);
 
 __host__ __device__ inline int colpack_offset(int n, int j) { return j * (n + 1) - (j * (j - 1)) / 2; }
-// Tile kernel factor: zero-padded r8 x r8 (r8 = n rounded up to kTileRows),
-// stored as 8-row x 4-column blocks, row block major: block (i / 8, j / 4) is
-// 32 contiguous floats (row i % 8, column j % 4), so one K step of a row
-// block is two 64-byte scalar loads.
-__host__ __device__ inline size_t l32_offset(int r8, int i, int j) {
-  return ((((size_t)(i >> 3) * (size_t)(r8 >> 2) + (size_t)(j >> 2)) * 8 + (i & 7)) << 2) + (j & 3);
-}
 __host__ __device__ inline size_t colpack_size(int n) { return (size_t)colpack_offset(n, n); }
 
 }  // namespace mcr

@@ -5,6 +5,8 @@
 #include <float.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "mcr_internal.h"
 #include "mcr_rng.h"
 
@@ -320,6 +322,13 @@ typedef void (*PathKernel)(PathArgs);
 PathKernel reg_kernel(int n);          // mcr_reg.hip
 PathKernel wave_kernel(int T);         // mcr_wave.hip
 PathKernel mfma_kernel(int n, int T);  // mcr_mfma.hip
+// mcr_f32.hip: kernel, waves per workgroup, workgroups per CU, dynamic LDS
+struct F32Shape {
+  PathKernel kernel;
+  int waves, per_cu;
+  size_t lds;
+};
+F32Shape f32_shape(int n);
 PathKernel mfma_big_kernel(int T);     // mcr_mfma_big.hip
 
 }  // namespace mcr

@@ -43,20 +43,21 @@ extern "C" {
 #define MCR_MAX_N_NOALLOC 608 /* largest through mcr_run_noalloc */
 
 /* precision / kernel family */
-#define MCR_PREC_FP32 0   /* fused fp32 VALU kernels: bit-exact with the C mirror */
+#define MCR_PREC_FP32 0   /* fp32 kernels: bit-exact with the C mirror */
 #define MCR_PREC_BF16X3 1 /* MFMA bf16 hi/lo split products, fp32 accumulation */
 #define MCR_PREC_AUTO 2   /* fastest supported for the size */
 
 /* explicit kernel override (0 = choose from precision) */
 #define MCR_KERNEL_AUTO 0
-#define MCR_KERNEL_VALU_REG 1  /* one path per lane, rows in registers, n <= 64 */
-#define MCR_KERNEL_VALU_TILE 2 /* 64 paths per workgroup, normals in LDS, n <= 608 */
+#define MCR_KERNEL_VALU_REG 1  /* fp32, one path per lane, rows in registers, n <= 64 */
+#define MCR_KERNEL_VALU_TILE 2 /* fp32 on the fp32 MFMA instructions (the same bits), n <= 608:
+                                  per wave up to 127 assets, normals in LDS above */
 #define MCR_KERNEL_MFMA 3      /* 64 paths per wave on 32x32x16 bf16 MFMA, n <= 127 */
 #define MCR_KERNEL_MFMA_LDS 4  /* 64 paths per workgroup, normals staged in LDS, n <= 767
                                   (24 row tiles) */
-#define MCR_KERNEL_VALU_CHUNK 5 /* fp32, 64 paths per workgroup, normals in 512-column LDS
-                                   chunks, any n <= 1024: fp32 queries past 608, and every
-                                   precision past 767 */
+#define MCR_KERNEL_VALU_CHUNK 5 /* the LDS form of kernel 2 for any n <= 1024 (past 608 its
+                                   normals are taken in 512-column LDS chunks): fp32 queries
+                                   past 608, and every precision past 767 */
 
 /* flags */
 #define MCR_F_VAR 0x1   /* portfolio-loss quantiles (VaR) and tail sums at alpha[] */

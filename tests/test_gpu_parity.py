@@ -140,6 +140,15 @@ def test_wave_kernel_exact(mcr, orc, n):
     assert r.kernel == "valu_tile"
 
 
+@pytest.mark.parametrize("kernel", [2, 5])
+@pytest.mark.parametrize("n", [128, 148, 149, 160, 308, 309, 320, 511, 512, 513, 608])
+def test_lds_kernel_exact_at_shape_edges(mcr, orc, n, kernel):
+    """The fp32 LDS kernel at the edges of its workgroup shapes (n = 148 / 149,
+    308 / 309), row tiles and column chunk, with and without a spare row for
+    the loss, over paths whose ids cross 2^32 inside a 64-path group."""
+    _exact_case(mcr, orc, n, 1500, max(1, n // 5), kernel, path_offset=2**32 - 741)
+
+
 @pytest.mark.parametrize("n", [1, 5, 9, 50, 129, 257, 600, 608, 609, 700, 1000, 1024])
 def test_chunk_kernel_exact(mcr, orc, n):
     """The column-chunk kernel (any n <= 1024; fp32 past 608): per-path
