@@ -30,11 +30,14 @@
 namespace mcr {
 
 // ---------------------------------------------------------------------------
-// Factor: FP64 Cholesky of A + delta I on one workgroup of 16 waves (blocked,
-// right-looking; see cholesky_body), then the portfolio moments.
+// Factor: FP64 Cholesky of A + delta I, then the portfolio moments.
 // Jitter policy: delta_0 = 0, delta_t = mean(diag) 10^(t-12) for t = 1..8, then
 // the modified factorisation with failing pivots clamped to delta_8.  A pivot
 // fails when it is not above n eps (A_jj + delta).
+// The first attempt runs on many workgroups, one launch per 32 columns
+// (k_chol_step); the rare retries, and the report of non-finite input, are the
+// finishing kernel's, on one workgroup (cholesky_body), with the same arithmetic
+// in the same order.
 // ---------------------------------------------------------------------------
 __device__ double block_sum_f64(double v, double* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -48,6 +51,8 @@ __device__ double block_sum_f64(double v, double* red) {
   return s;
 }
 
+// Retries (attempts 2 to 10) of a factorisation whose first attempt failed, or
+// the rejection of non-finite input.
 // FP64 Cholesky of A + delta I into L (row-major, zero upper triangle) on one
 // workgroup of 1024 threads, right-looking by panels of kPanel columns:
 //   panel:    thread r holds row k0 + r of the panel in registers; column c is
@@ -56,8 +61,8 @@ __device__ double block_sum_f64(double v, double* red) {
 //             pivot, scales its entry and updates its later panel columns;
 //   trailing: A22 -= L21 L21^T on the lower triangle, 4 x 4 register tiles
 //             read from a column-major LDS copy of the panel.
-// Jitter policy: attempt t adds delta_t = mean(diag A) * 10^(min(t,8)-12)
-// (t >= 1); attempt 9 clamps failing pivots to delta.  A pivot fails when it
+// Jitter policy: try t = 1..9 adds delta_t = mean(diag A) * 10^(min(t,8)-12);
+// try 9 clamps failing pivots to delta.  A pivot fails when it
 // is not above n eps (A_jj + delta).  Returns false (and records attempts =
 // -1) for non-finite A.
 constexpr int kPanel = 16;
@@ -102,9 +107,9 @@ __device__ bool cholesky_body(const FactorArgs& a, FactorShared<MAXN>& sh, int* 
 
   int attempts = 0, clamped = 0, fail = 0, last_fail = 0;
   double delta = 0.0;
-  for (int t = 0; t <= 9; ++t) {
+  for (int t = 1; t <= 9; ++t) {
     const bool clamp = (t == 9);
-    delta = (t == 0) ? 0.0 : mean * pow(10.0, (double)((t < 8 ? t : 8) - 12));
+    delta = mean * pow(10.0, (double)((t < 8 ? t : 8) - 12));
     fail = 0;
     clamped = 0;
     for (int i = wave; i < n; i += nwave)
@@ -223,19 +228,33 @@ __device__ bool cholesky_body(const FactorArgs& a, FactorShared<MAXN>& sh, int* 
   return true;
 }
 
+// v_j = sum_{i >= j} L_ij w_i, i ascending; the loads of 32 rows are in flight
+// together (one at a time cost a memory latency per row).
+__device__ __forceinline__ double loading_of(const FactorArgs& a, int j) {
+  const int n = a.n;
+  const double* __restrict__ col = a.L + j;
+  double s = 0.0;
+  int i = j;
+  for (; i + 32 <= n; i += 32) {
+    double l[32];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) l[u] = col[(size_t)(i + u) * n];
+#pragma unroll
+    for (int u = 0; u < 32; ++u) s += l[u] * a.w[i + u];
+  }
+  for (; i < n; ++i) s += col[(size_t)i * n] * a.w[i];
+  return s;
+}
+
 // Portfolio loading v = L^T w, mean w^T mu and sd ||v|| in FP64, and the
 // query's record (factor outcome, moments, VaR windows).
-__device__ void moments_body(const FactorArgs& a, double* red, int attempts, int clamped,
+// The columns before j0 have their v_j already.
+__device__ void moments_body(const FactorArgs& a, double* red, int j0, int attempts, int clamped,
                              int last_fail, double delta) {
   const int n = a.n;
   const int tid = threadIdx.x;
-  const double* __restrict__ L = a.L;
   __syncthreads();
-  for (int j = tid; j < n; j += blockDim.x) {
-    double s = 0.0;
-    for (int i = j; i < n; ++i) s += L[(size_t)i * n + j] * a.w[i];
-    a.v64[j] = s;
-  }
+  for (int j = j0 + tid; j < n; j += blockDim.x) a.v64[j] = loading_of(a, j);
   __syncthreads();
   double mp = 0.0, ss = 0.0;
   for (int i = tid; i < n; i += blockDim.x) {
@@ -268,8 +287,253 @@ __device__ void moments_body(const FactorArgs& a, double* red, int attempts, int
 }
 
 
+// ---------------------------------------------------------------------------
+// First attempt, launch s of ceil(n / 32): block column s (columns 32s .. 32s +
+// 31) is finished and the columns right of it take the update of block column
+// s - 1, which only needs what launch s - 1 left behind:
+//   panel waves   rows 0-31 of the wave's 64 are the diagonal block (every wave
+//                 factors it for itself: no exchange, no barrier), rows 32-63 its
+//                 own 32 rows below.  A lane holds its row's 32 entries, takes
+//                 block column s - 1's update and then the 32 columns, the
+//                 pivots and the diagonal block's entries coming by readlane.
+//   update tiles  64 x 64, block column s - 1's product subtracted;
+//   loading       block column s - 1's part of v = L^T w, a column per lane.
+// Every entry sees the operations of a right-looking factorisation by panels of
+// 16 columns in its order (per panel a chain of 16 fused multiply-adds from zero,
+// then one subtraction; inside a panel one fused multiply-add per column), so L
+// has the bits that cholesky_body's algorithm gives it.
+// Bound: the chain of 32 square roots and reciprocals of a launch (about 8 of its
+// 21 us; its loads and stores cross the XCDs' caches).  Factor and layouts at n =
+// 50 / 143 / 301 / 600 / 1024: 52 / 133 / 263 / 414 / 773 us; one workgroup did the
+// whole of it before in 67 / 163 / 460 / 1809 / 6768.
+// ---------------------------------------------------------------------------
+constexpr int kBlk = 32;
+
+// double of lane `src` (a constant) in every lane
+__device__ __forceinline__ double bcast(double v, int src) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, src);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), src);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+struct CholShared {
+  union {
+    struct {
+      double prev[kBlk][kBlk];       // L[diagonal block's rows][block column s - 1]
+      double cross[4][kPanel][kPanel];  // per wave: rows 16-31 of the diagonal block, first panel
+    } p;
+    struct {
+      double a[kBlk][68], b[kBlk][68];  // [column of s - 1][row of the tile]
+    } u;
+  };
+  int failed;
+} __attribute__((aligned(16)));
+
+__device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) {
+  const int n = a.n, k0 = kBlk * s, kb = min(kBlk, n - k0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31;
+  const bool diag = lane < 32;
+  const int row = diag ? k0 + r : k0 + kBlk * (1 + 4 * blk + wave) + r;
+  const bool valid = row < n;
+  const double* __restrict__ src = s <= 1 ? a.A : a.L;
+  double* __restrict__ L = a.L;
+  double x[kBlk];
+#pragma unroll
+  for (int c = 0; c < kBlk; ++c)
+    x[c] = valid && c < kb && (!diag || c <= r) ? src[(size_t)row * n + k0 + c]
+                                                : (diag && c == r ? 1.0 : 0.0);  // identity pads
+  if (s > 0) {
+    const int kp = k0 - kBlk;
+    for (int e = threadIdx.x; e < kBlk * kBlk; e += blockDim.x) {
+      const int j = e / kBlk, p = e % kBlk;
+      sh.p.prev[j][p] = k0 + j < n ? L[(size_t)(k0 + j) * n + kp + p] : 0.0;
+    }
+    double lp[kBlk];
+#pragma unroll
+    for (int p = 0; p < kBlk; ++p) lp[p] = valid ? L[(size_t)row * n + kp + p] : 0.0;
+    __syncthreads();
+    // four columns at a time: eight independent chains keep the unit busy
+#pragma unroll
+    for (int j = 0; j < kBlk; j += 4) {
+      double acc[4][2] = {};
+#pragma unroll
+      for (int p = 0; p < kPanel; ++p)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          acc[u][0] = fma(lp[p], sh.p.prev[j + u][p], acc[u][0]);
+          acc[u][1] = fma(lp[kPanel + p], sh.p.prev[j + u][kPanel + p], acc[u][1]);
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[j + u] = x[j + u] - acc[u][0] - acc[u][1];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  double piv = 0.0;  // this lane's pivot, as its column found it
+#pragma unroll
+  for (int q = 0; q < kBlk; q += kPanel) {
+#pragma unroll
+    for (int c = q; c < q + kPanel; ++c) {
+      const double d = bcast(x[c], c);
+      if (lane == c) piv = d;
+      const double ljj = sqrt(d), rl = 1.0 / ljj;
+      const double lr = x[c] * rl;
+      x[c] = lane == c ? ljj : lr;
+#pragma unroll
+      for (int c2 = c + 1; c2 < q + kPanel; ++c2) x[c2] = fma(-lr, bcast(lr, c2), x[c2]);
+    }
+    if (q == 0) {
+      // the first panel's update of the second's columns
+      if (diag && r >= kPanel) {
+#pragma unroll
+        for (int p = 0; p < kPanel; ++p) sh.p.cross[wave][r - kPanel][p] = x[p];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int c = 0; c < kPanel; ++c) {
+        double acc = 0.0;
+#pragma unroll
+        for (int p = 0; p < kPanel; ++p) acc = fma(x[p], sh.p.cross[wave][c][p], acc);
+        x[kPanel + c] -= acc;
+      }
+    }
+  }
+  const bool first = blk == 0 && wave == 0;
+  if (valid && (!diag || first)) {
+#pragma unroll
+    for (int c = 0; c < kBlk; ++c)
+      if (c < kb) L[(size_t)row * n + k0 + c] = diag && c > r ? 0.0 : x[c];
+  }
+  if (first) {
+    const double ajj = diag && valid ? a.A[(size_t)row * n + row] : 1.0;
+    const double tol = (double)n * DBL_EPSILON * ajj;
+    const unsigned long long bad = __ballot(diag && r < kb && (!(piv > tol) || !isfinite(piv)));
+    const int fail = bad ? k0 + __ffsll((long long)bad) : 0;  // first failing column + 1
+    if (lane == 0 && (s == 0 || fail)) a.info->fail_col = fail;
+  }
+}
+
+// The tile at (r0, c0) of the lower triangle takes block column kp's update.
+__device__ void chol_update(const FactorArgs& a, int s, int r0, int c0, CholShared& sh) {
+  const int n = a.n, kp = kBlk * (s - 1);
+  const double* __restrict__ src = s == 1 ? a.A : a.L;
+  double* __restrict__ L = a.L;
+  for (int e = threadIdx.x; e < 64 * kBlk; e += blockDim.x) {
+    const int i = e / kBlk, p = e % kBlk;
+    sh.u.a[p][i] = r0 + i < n ? L[(size_t)(r0 + i) * n + kp + p] : 0.0;
+    sh.u.b[p][i] = c0 + i < n ? L[(size_t)(c0 + i) * n + kp + p] : 0.0;
+  }
+  const int ri = 4 * (threadIdx.x >> 4), cj = 4 * (threadIdx.x & 15);
+  double x[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = r0 + ri + u, j = c0 + cj + v;
+      x[u][v] = i < n && j <= i ? src[(size_t)i * n + j] : 0.0;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < kBlk; h += kPanel) {
+    double acc[4][4] = {};
+#pragma unroll 4
+    for (int p = h; p < h + kPanel; ++p) {
+      const double2* pa = (const double2*)&sh.u.a[p][ri];
+      const double2* pb = (const double2*)&sh.u.b[p][cj];
+      const double2 a01 = pa[0], a23 = pa[1], b01 = pb[0], b23 = pb[1];
+      const double av[4] = {a01.x, a01.y, a23.x, a23.y};
+      const double bv[4] = {b01.x, b01.y, b23.x, b23.y};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[u][v] = fma(av[u], bv[v], acc[u][v]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[u][v] -= acc[u][v];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = r0 + ri + u, j = c0 + cj + v;
+      if (i < n && j <= i) L[(size_t)i * n + j] = x[u][v];
+    }
+}
+
+// Launch 0 beside the first panel: the zero upper triangle of L, and the search
+// of A's for non-finite entries (the factorisation itself meets those of the
+// lower one).  One found poisons A's first entry, which the finishing kernel
+// tests.
+__device__ void chol_upper(const FactorArgs& a, int r0, int c0) {
+  const int n = a.n;
+  bool bad = false;
+  for (int e = threadIdx.x; e < 64 * 64; e += blockDim.x) {
+    const int i = r0 + e / 64, j = c0 + e % 64;
+    if (i < n && j < n && j > i) {
+      bad |= !isfinite(a.A[(size_t)i * n + j]);
+      a.L[(size_t)i * n + j] = 0.0;
+    }
+  }
+  if (bad) const_cast<double*>(a.A)[0] = __builtin_nan("");
+}
+
+__host__ __device__ inline int chol_panel_wgs(int n, int s) {
+  const int below = n - kBlk * (s + 1);  // rows under the diagonal block, 128 per workgroup
+  return below > 0 ? (below + 127) / 128 : 1;
+}
+__host__ __device__ inline int chol_step_wgs(int n, int s) {
+  if (kBlk * s >= n) return 0;
+  const int t = s == 0 ? (n + 63) / 64 : (n - kBlk * (s + 1) + 63) / 64;
+  return chol_panel_wgs(n, s) + (t > 0 ? (s == 0 ? t * t : t * (t + 1) / 2) : 0) + (s > 0 ? 1 : 0);
+}
+
+__device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
+  const int n = a.n, np = chol_panel_wgs(n, s);
+  if ((int)blockIdx.x >= chol_step_wgs(n, s) || a.reuse) return;
+  if (s > 0) {
+    // one read for the workgroup: the first one may be writing it
+    if (threadIdx.x == 0) sh.failed = a.info->fail_col;
+    __syncthreads();
+    if (sh.failed != 0) return;  // a retry follows
+  }
+  if ((int)blockIdx.x < np) {
+    chol_panel(a, s, blockIdx.x, sh);
+    return;
+  }
+  if (s == 0) {
+    const int t = blockIdx.x - np, nt = (n + 63) / 64;
+    chol_upper(a, 64 * (t / nt), 64 * (t % nt));
+    return;
+  }
+  if ((int)blockIdx.x == np) {
+    const int j = kBlk * (s - 1) + threadIdx.x;
+    if (threadIdx.x < kBlk) a.v64[j] = loading_of(a, j);
+    return;
+  }
+  const int t = blockIdx.x - np - 1;
+  int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (bi * (bi + 1) / 2 > t) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
+  const int bj = t - bi * (bi + 1) / 2, o = kBlk * (s + 1);
+  chol_update(a, s, o + 64 * bi, o + 64 * bj, sh);
+}
+
+__global__ __launch_bounds__(256) void k_chol_step(FactorArgs a, int s) {
+  __shared__ CholShared sh;
+  chol_step(a, s, sh);
+}
+// blockIdx.y = query of a batch
+__global__ __launch_bounds__(256) void k_chol_step_batch(const FactorArgs* fas, int s) {
+  __shared__ CholShared sh;
+  const FactorArgs a = fas[blockIdx.y];
+  chol_step(a, s, sh);
+}
+
 template <int MAXN>
-__device__ void factor_body(const FactorArgs& a, FactorShared<MAXN>& sh) {
+__device__ void factor_finish(const FactorArgs& a, FactorShared<MAXN>& sh) {
   const int tid = threadIdx.x;
 
   // Clear the query's accumulators.
@@ -279,8 +543,9 @@ __device__ void factor_body(const FactorArgs& a, FactorShared<MAXN>& sh) {
   }
   for (int i = tid; i < kHistBins; i += blockDim.x) a.hist[i] = 0u;
 
-  int attempts = 0, clamped = 0, last_fail = 0;
+  int attempts = 1, clamped = 0, last_fail = 0;
   double delta = 0.0;
+  int j0 = 0;
   if (a.reuse) {
     // L holds this covariance's factor from an earlier launch.
     const DevInfo fi = *a.finfo;
@@ -297,8 +562,11 @@ __device__ void factor_body(const FactorArgs& a, FactorShared<MAXN>& sh) {
       }
       return;
     }
-  } else if (!cholesky_body(a, sh, &attempts, &clamped, &last_fail, &delta)) {
-    return;
+  } else if (a.info->fail_col != 0 || !isfinite(a.A[0])) {
+    __syncthreads();  // the record is read before anyone writes it
+    if (!cholesky_body(a, sh, &attempts, &clamped, &last_fail, &delta)) return;
+  } else {
+    j0 = kBlk * ((a.n - 1) / kBlk);  // the launches left the last block column
   }
   if (a.finfo && !a.reuse && tid == 0) {
     a.finfo->attempts = attempts;
@@ -306,13 +574,13 @@ __device__ void factor_body(const FactorArgs& a, FactorShared<MAXN>& sh) {
     a.finfo->fail_col = last_fail;
     a.finfo->jitter = delta;
   }
-  moments_body(a, sh.red, attempts, clamped, last_fail, delta);
+  moments_body(a, sh.red, j0, attempts, clamped, last_fail, delta);
 }
 
 template <int MAXN>
 __global__ __launch_bounds__(1024) void k_factor(FactorArgs a) {
   __shared__ FactorShared<MAXN> sh;
-  factor_body(a, sh);
+  factor_finish(a, sh);
 }
 
 // One workgroup per query of a batch (n <= MAXN).
@@ -320,11 +588,13 @@ template <int MAXN>
 __global__ __launch_bounds__(1024) void k_factor_batch(const FactorArgs* fas) {
   __shared__ FactorShared<MAXN> sh;
   const FactorArgs a = fas[blockIdx.x];
-  factor_body(a, sh);
+  factor_finish(a, sh);
 }
 
 hipError_t launch_factor(const FactorArgs& a, hipStream_t stream) {
   if (a.n < 1 || a.n > kChunkMaxN) return hipErrorInvalidValue;
+  for (int s = 0; kBlk * s < a.n; ++s)
+    hipLaunchKernelGGL(k_chol_step, dim3(chol_step_wgs(a.n, s)), dim3(256), 0, stream, a, s);
   if (a.n <= kMaxN)
     hipLaunchKernelGGL(k_factor<kMaxN>, dim3(1), dim3(1024), 0, stream, a);
   else
@@ -336,6 +606,8 @@ hipError_t launch_factor(const FactorArgs& a, hipStream_t stream) {
 // up to kBatchMaxN)
 hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStream_t stream) {
   if (max_n < 1 || max_n > kBatchMaxN) return hipErrorInvalidValue;
+  for (int s = 0; kBlk * s < max_n; ++s)
+    hipLaunchKernelGGL(k_chol_step_batch, dim3(chol_step_wgs(max_n, s), nq), dim3(256), 0, stream, fas, s);
   if (max_n <= kMaxN)
     hipLaunchKernelGGL(k_factor_batch<kMaxN>, dim3(nq), dim3(1024), 0, stream, fas);
   else

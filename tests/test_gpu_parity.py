@@ -71,6 +71,45 @@ def test_factor_jitter_policy_matches_oracle(mcr, orc):
     assert np.allclose(L, oL, rtol=1e-8, atol=1e-12)
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 96, 97, 127, 128, 129, 160,
+                               161, 288, 289, 767, 1024])
+def test_factor_at_block_edges(mcr, n):
+    """L L^T = A at the edges of the factor's 16-column panels, 32-column
+    launches, 128-row workgroups and 64 x 64 update tiles.  Each entry's sum of
+    at most n products and the factor's own rounding stay within (n + 10) eps
+    of sqrt(A_ii A_jj) (the standard bound for Cholesky)."""
+    A = random_spd(n, 100 + n, cond=50.0)
+    L, att, jit, cl = mcr.factor(A)
+    assert (att, jit, cl) == (1, 0.0, 0)
+    assert np.all(np.triu(L, 1) == 0) and np.all(np.diag(L) > 0)
+    d = np.sqrt(np.diag(A))
+    assert np.max(np.abs(L @ L.T - A) / np.outer(d, d)) <= 2 * (n + 10) * np.finfo(float).eps
+
+
+@pytest.mark.parametrize("col", [0, 1, 15, 16, 31, 32, 33, 63, 64, 95, 96, 100])
+def test_factor_retries_from_any_column(mcr, orc, col):
+    """A pivot that fails in any column of any launch sends the factor through
+    the jitter policy, with the oracle's decisions; a non-finite entry in either
+    triangle is refused."""
+    # positive semidefinite: asset col's factor row is a mixture of the earlier
+    # ones, so its pivot is rounding noise (exactly 0 for col = 0) and the first
+    # jitter step makes it positive
+    A = random_spd(101, 7, cond=10.0)
+    F = np.linalg.cholesky(A)
+    F[col] = np.random.default_rng(col).dirichlet(np.ones(col)) @ F[:col] if col else 0.0
+    B = F @ F.T
+    L, att, jit, cl = mcr.factor(B)
+    oatt, oL, ojit, ocl = orc.factor(B)
+    assert (att, cl) == (oatt, ocl) and att == 2
+    assert jit == pytest.approx(ojit, rel=1e-13)
+    for i, j in ((col, 100), (100, col)):
+        C = A.copy()
+        C[i, j] = np.nan
+        with pytest.raises(mcr.McrError) as e:
+            mcr.factor(C)
+        assert e.value.code == mcr.MCR_E_FACTOR
+
+
 def test_factor_clamp_fallback(mcr, orc):
     A = np.diag([1.0, 1.0, -0.5, 1.0]) * 1e-4
     L, att, jit, cl = mcr.factor(A)
