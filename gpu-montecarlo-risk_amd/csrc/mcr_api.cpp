@@ -882,6 +882,12 @@ int class_grid(BatchKernel k, int block) {
   return resident_blocks(reinterpret_cast<const void*>(k), block) * cus;
 }
 
+uint64_t item_groups(int n, uint64_t groups, int grid, uint64_t cap) {
+  uint64_t g = groups / (4 * (uint64_t)grid);
+  if (n <= kSmallMaxN) g = std::max<uint64_t>(4, g / 4 * 4);
+  return std::max<uint64_t>(1, std::min(g, cap));
+}
+
 void order_by_class(std::vector<WorkItem>* items, const std::vector<BatchKernel>& qk,
                     const std::vector<int>& qb, const std::vector<double>& qcost, bool lpt,
                     std::vector<ClassRun>* runs) {
@@ -1098,8 +1104,7 @@ int plan_batch(const mcr_query* qs, int nq, int chunk_paths, int order, const in
     bp->na[i] = (q->flags & MCR_F_VAR) ? q->n_alpha : 0;
     bp->max_n = std::max(bp->max_n, q->n);
   }
-  // work items: per class, runs of cg groups, with at least four items per
-  // resident workgroup (small classes: per wave) so the class's launch balances
+  // work items: per class, runs of at most cg groups
   std::vector<BatchKernel> qk(nq);
   std::vector<int> qb(nq);
   std::vector<double> qcost(nq);
@@ -1113,8 +1118,7 @@ int plan_batch(const mcr_query* qs, int nq, int chunk_paths, int order, const in
   const uint64_t cg = (uint64_t)std::max(1, chunk_paths / 64);
   bp->items.clear();
   for (int i = 0; i < nq; ++i) {
-    const uint64_t slots = (uint64_t)class_grid(qk[i], qb[i]) * (qs[i].n <= kSmallMaxN ? 4 : 1);
-    const uint64_t cgi = std::max<uint64_t>(1, std::min(cg, class_groups[qk[i]] / (4 * slots)));
+    const uint64_t cgi = item_groups(qs[i].n, class_groups[qk[i]], class_grid(qk[i], qb[i]), cg);
     const uint64_t G = ((uint64_t)qs[i].paths + 63) / 64;
     for (uint64_t f = 0; f < G; f += cgi) {
       WorkItem w;

@@ -632,12 +632,10 @@ int mcr_server::plan_round(uint64_t round, RoundRec* rr, std::vector<WorkItem>* 
     total_units += (double)g * c;
     grant.push_back({j, g});
   }
-  // Item size per kernel class, as batches size them: at least four items
-  // per resident slot of the class's launch (a workgroup; a wave for the
-  // small-n classes, whose waves take items on their own) and at most
-  // kItemGroups groups.  Sizing from the round's total instead gave a class
-  // with little work a few huge items, one wave or workgroup grinding through
-  // each while the rest of the device idled inside that launch.
+  // Item size per kernel class, as batches size them (item_groups).  Sizing from
+  // the round's total instead gave a class with little work a few huge items,
+  // one workgroup grinding through each while the rest of the device idled
+  // inside that launch.
   // One snapshot of the tuned workgroup shapes for the whole round: the batch
   // autotuner may change them from another thread, and a class's kernel and
   // its block size must come from the same shape.
@@ -645,16 +643,14 @@ int mcr_server::plan_round(uint64_t round, RoundRec* rr, std::vector<WorkItem>* 
   tuned_shapes(shapes);
   std::map<BatchKernel, uint64_t> class_groups;
   for (auto& gr : grant) class_groups[class_kernel(gr.first->q.n, shapes)] += gr.second;
-  auto item_groups = [&](const Job* j) {
+  auto job_item_groups = [&](const Job* j) {
     const int n = j->q.n;
     const BatchKernel k = class_kernel(n, shapes);
-    const uint64_t slots =
-        (uint64_t)class_grid(k, class_block(n, shapes)) * (n <= kSmallMaxN ? 4 : 1);
-    return std::max<uint64_t>(1, std::min<uint64_t>(kItemGroups, class_groups[k] / (4 * slots)));
+    return item_groups(n, class_groups[k], class_grid(k, class_block(n, shapes)), kItemGroups);
   };
   size_t est = 0;
   for (auto& gr : grant) {
-    const uint64_t ig = item_groups(gr.first);
+    const uint64_t ig = job_item_groups(gr.first);
     est += (size_t)((gr.second + ig - 1) / ig);
   }
   const double scale = est > kMaxItems ? (double)est / kMaxItems + 1.0 : 1.0;
@@ -662,7 +658,7 @@ int mcr_server::plan_round(uint64_t round, RoundRec* rr, std::vector<WorkItem>* 
   for (auto& gr : grant) {
     Job* j = gr.first;
     const double c = group_cost(j->T, j->S);
-    const uint64_t ig = std::max<uint64_t>(1, (uint64_t)std::ceil(scale * (double)item_groups(j)));
+    const uint64_t ig = std::max<uint64_t>(1, (uint64_t)std::ceil(scale * (double)job_item_groups(j)));
     const uint64_t g0 = j->next_group, g1 = g0 + gr.second;
     for (uint64_t g = g0; g < g1; g += ig) {
       WorkItem w;

@@ -94,6 +94,17 @@ def test_chunking_and_order_do_not_change_results(mcr, chunk, order):
         same(x, y)
 
 
+@pytest.mark.parametrize("chunk,grid", [(64, 1), (192, 1), (320, 3), (2048, 0)])
+def test_small_items_over_the_workgroup(mcr, chunk, grid):
+    """Items of one group, fewer and more groups than waves, and a ragged last
+    one, on one workgroup (every later item from the counter), three, and the
+    default grid (first items by workgroup index)."""
+    ps = portfolios(8, sizes=(1, 31, 32, 63, 95, 127), paths=[64, 63, 321, 1000, 4097, 40001])
+    res, _ = mcr.run_batch(ps, use_graph=False, chunk_paths=chunk, grid=grid)
+    for p, r in zip(ps, res):
+        same(r, alone(mcr, p))
+
+
 def test_batch_refinement_fallback(mcr):
     ps = portfolios(5, sizes=(20, 40))
     ps[1]["alphas"] = (0.95, 0.99)
