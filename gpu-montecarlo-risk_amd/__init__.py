@@ -235,8 +235,8 @@ def _make_query(mu, sigma, x, k, paths, seed, weights=None, precision=PREC_FP32,
     w = None if weights is None else np.ascontiguousarray(weights, dtype=np.float64)
     if w is not None and w.shape != (n,):
         raise ValueError(f"weights must have shape ({n},), not {w.shape}")
-    S = np.zeros(paths, dtype=np.int32) if want_S else None
-    loss = np.zeros(paths, dtype=np.float32) if want_loss else None
+    S = np.empty(paths, dtype=np.int32) if want_S else None
+    loss = np.empty(paths, dtype=np.float32) if want_loss else None
     hist = np.zeros(n + 1, dtype=np.int64) if want_hist else None
     flags = extra_flags
     if alphas:
@@ -483,7 +483,7 @@ def factor(sigma):
     """GPU FP64 Cholesky with the jitter policy: (L, attempts, jitter, clamped)."""
     sigma = _square(sigma)
     n = sigma.shape[0]
-    L = np.zeros((n, n), dtype=np.float64)
+    L = np.empty((n, n), dtype=np.float64)
     info = FactorInfo()
     _check(lib().mcr_factor(n, _ptr(sigma, _f64p), n, _ptr(L, _f64p), ctypes.byref(info)))
     return L, info.attempts, info.jitter, info.clamped

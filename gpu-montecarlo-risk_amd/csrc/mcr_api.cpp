@@ -87,6 +87,7 @@ int ensure_init(int device) {
   HIP_TRY(hipEventCreate(&g_ctx.ev0));
   HIP_TRY(hipEventCreate(&g_ctx.ev1));
   HIP_TRY(hipEventCreate(&g_ctx.evs));
+  for (hipEvent_t& e : g_ctx.evc) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   MCR_TRY(create_forks(&g_ctx.forks, kMaxForks));
   // the scratch array's address on this device (the device is current)
   void* sp = nullptr;
@@ -333,17 +334,67 @@ int validate(const mcr_query* q) {
   return MCR_OK;
 }
 
+// Pinned staging of a query: the image of its inputs (A, mu, w as the device lays
+// them out), what k_collect writes, and the two buffers of copy_out.
+struct HostBuffers {
+  double *A, *mu, *w;
+  DevInfo* info;
+  DevAccum* acc;
+  unsigned long long* s_hist;
+  unsigned cap;  // losses per window
+  float* win;    // [n_alpha][cap]
+  char* piece[2];
+};
+
 struct Staged {
   Plan plan;
   DevBuffers d;
+  HostBuffers h;
   char* host;  // pinned staging; nullptr in the allocation-free mode
 };
 
-// Uploads inputs, factors and prepares on the device.  Leaves the context
-// locked state untouched; caller holds g_mu.  With noalloc the device buffers
-// are carved from the scratch array and the inputs are copied straight from
-// the caller's arrays (no arena growth, no pinned staging).
-int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noalloc = false) {
+// Device memory to the caller's array on the query's stream, through the pinned
+// pieces: one is copied out while the next one arrives (the runtime stages a
+// copy to pageable memory in pieces one after the other).  Once the first piece
+// is in, ok() decides whether the caller's array is written at all.  The copy out,
+// bound by the first touch of the caller's pages, is no faster on four threads and
+// slower on eight.
+constexpr size_t kPieceBytes = 1u << 20;
+template <typename F>
+int copy_out(const Staged& st, void* dst, const void* dev, size_t bytes, F ok) {
+  if (!st.host) {
+    HIP_TRY(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, g_ctx.stream));
+    HIP_TRY(hipStreamSynchronize(g_ctx.stream));
+    return MCR_OK;
+  }
+  const size_t np = (bytes + kPieceBytes - 1) / kPieceBytes;
+  auto fetch = [&](size_t i) {
+    const size_t off = i * kPieceBytes;
+    HIP_TRY(hipMemcpyAsync(st.h.piece[i & 1], (const char*)dev + off,
+                           std::min(kPieceBytes, bytes - off), hipMemcpyDeviceToHost, g_ctx.stream));
+    HIP_TRY(hipEventRecord(g_ctx.evc[i & 1], g_ctx.stream));
+    return (int)MCR_OK;
+  };
+  for (size_t i = 0; i < std::min<size_t>(np, 2); ++i) MCR_TRY(fetch(i));
+  for (size_t i = 0; i < np; ++i) {
+    HIP_TRY(hipEventSynchronize(g_ctx.evc[i & 1]));
+    if (const int r = i == 0 ? ok() : MCR_OK) {
+      HIP_TRY(hipStreamSynchronize(g_ctx.stream));  // the second piece may be on its way
+      return r;
+    }
+    const size_t off = i * kPieceBytes;
+    std::memcpy((char*)dst + off, st.h.piece[i & 1], std::min(kPieceBytes, bytes - off));
+    if (i + 2 < np) MCR_TRY(fetch(i + 2));
+  }
+  return MCR_OK;
+}
+
+// Uploads inputs, factors and prepares on the device (prep = false: factors
+// only).  Leaves the context locked state untouched; caller holds g_mu.  With
+// noalloc the device buffers are carved from the scratch array and the inputs are
+// copied straight from the caller's arrays (no arena growth, no pinned staging).
+int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noalloc = false,
+                bool prep = true) {
   Plan& p = st->plan;
   p.n = q->n;
   MCR_TRY(choose_kernel(q, &p));
@@ -384,31 +435,47 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   } else {
     MCR_TRY(reserve_arena(dev_bytes));
     layout(p, (char*)g_ctx.arena, &st->d);
-    const size_t in_bytes = align_up((n * n + 2 * n) * sizeof(double));
-    const size_t out_bytes = align_up(sizeof(DevInfo)) + align_up(sizeof(DevAccum)) +
-                             align_up(kHistBins * sizeof(unsigned)) +
-                             align_up((n + 1) * sizeof(unsigned long long));
-    MCR_TRY(reserve_host(in_bytes + out_bytes));
+    // the pieces of copy_out: per-path outputs, or the factor alone
+    const size_t piece_bytes = std::min(kPieceBytes, prep ? p.chunk * 4 : n * n * sizeof(double));
+    const unsigned cap = want_var_windows ? window_capacity(q, kGatherCap) : 0;
+    HostBuffers& h = st->h;
+    size_t in_bytes = 0;
+    auto carve = [&](char* base) {
+      Carver c{base};
+      h.A = c.take<double>(n * n);
+      h.mu = c.take<double>(n);
+      h.w = c.take<double>(n);
+      in_bytes = c.off;
+      h.info = c.take<DevInfo>(1);
+      h.acc = c.take<DevAccum>(1);
+      h.s_hist = c.take<unsigned long long>(n + 1);
+      h.cap = cap;
+      h.win = c.take<float>((size_t)p.n_alpha * cap);
+      for (char*& x : h.piece) x = c.take<char>(piece_bytes);
+      return c.off;
+    };
+    MCR_TRY(reserve_host(carve(nullptr)));
     st->host = (char*)g_ctx.host;
-    double* hA = (double*)st->host;
-    double* hmu = hA + n * n;
-    double* hw = hmu + n;
+    carve(st->host);
     for (size_t i = 0; i < n; ++i) {
-      std::memcpy(hA + i * n, q->sigma + i * (size_t)q->ld_sigma, n * sizeof(double));
-      hmu[i] = q->mu[i];
-      hw[i] = q->weights ? q->weights[i] : 1.0 / (double)n;
-    }
-    for (size_t i = 0; i < n; ++i)
-      if (!std::isfinite(hmu[i]) || !std::isfinite(hw[i])) {
+      h.mu[i] = q->mu[i];
+      h.w[i] = q->weights ? q->weights[i] : 1.0 / (double)n;
+      if (!std::isfinite(h.mu[i]) || !std::isfinite(h.w[i])) {
         set_error("mu or weights not finite at %zu", i);
         return MCR_E_ARG;
       }
-    HIP_TRY(hipMemcpyAsync(st->d.A, hA, n * n * sizeof(double), hipMemcpyHostToDevice,
-                           g_ctx.stream));
-    HIP_TRY(hipMemcpyAsync(st->d.mu, hmu, n * sizeof(double), hipMemcpyHostToDevice,
-                           g_ctx.stream));
-    HIP_TRY(hipMemcpyAsync(st->d.w, hw, n * sizeof(double), hipMemcpyHostToDevice,
-                           g_ctx.stream));
+    }
+    // The image goes up as it lies, in pieces: one is uploaded while the next is
+    // gathered.
+    size_t up = 0;
+    for (size_t i = 0; i < n; ++i) {
+      std::memcpy(h.A + i * n, q->sigma + i * (size_t)q->ld_sigma, n * sizeof(double));
+      const size_t have = i + 1 < n ? (i + 1) * n * sizeof(double) : in_bytes;
+      if (have - up < kPieceBytes && i + 1 < n) continue;
+      HIP_TRY(hipMemcpyAsync((char*)st->d.A + up, (char*)h.A + up, have - up,
+                             hipMemcpyHostToDevice, g_ctx.stream));
+      up = have;
+    }
   }
 
   FactorArgs fa = {};
@@ -424,7 +491,7 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   fa.hist = st->d.hist;
   HIP_TRY(hipEventRecord(g_ctx.evs, g_ctx.stream));
   HIP_TRY(launch_factor(fa, g_ctx.stream));
-  HIP_TRY(hipMemsetAsync(st->d.s_hist, 0, (n + 1) * sizeof(unsigned long long), g_ctx.stream));
+  if (!prep) return MCR_OK;
 
   PrepArgs pa = {};
   pa.L = st->d.L;
@@ -440,7 +507,28 @@ int stage_query(const mcr_query* q, Staged* st, bool want_var_windows, bool noal
   pa.v32 = st->d.v32;
   pa.lfrag = st->d.lfrag;
   pa.rowinit = st->d.rowinit;
+  pa.s_hist = (q->flags & MCR_F_SHIST) ? st->d.s_hist : nullptr;
   HIP_TRY(launch_prep(pa, g_ctx.stream));
+  return MCR_OK;
+}
+
+// The query's record (and with n_alpha its windows, with hist its S histogram) to
+// the pinned staging.
+int launch_report(const Staged& st, int n_alpha, bool hist) {
+  CollectArgs c = {};
+  c.info = st.d.info;
+  c.acc = st.d.acc;
+  c.gather = st.d.gather;
+  c.s_hist = hist ? st.d.s_hist : nullptr;
+  c.gather_cap = kGatherCap;
+  c.n = st.plan.n;
+  c.n_alpha = n_alpha;
+  c.cap = st.h.cap;
+  c.h_info = st.h.info;
+  c.h_acc = st.h.acc;
+  c.h_win = st.h.win;
+  c.h_hist = st.h.s_hist;
+  HIP_TRY(launch_collect(c, g_ctx.stream));
   return MCR_OK;
 }
 
@@ -451,15 +539,10 @@ int read_info(const Staged& st, DevInfo* info, DevAccum* acc) {
     HIP_TRY(hipStreamSynchronize(g_ctx.stream));
     return MCR_OK;
   }
-  char* out = st.host + align_up((size_t)st.plan.n * st.plan.n * sizeof(double) +
-                                 2 * (size_t)st.plan.n * sizeof(double));
-  DevInfo* hi = (DevInfo*)out;
-  DevAccum* ha = (DevAccum*)(out + align_up(sizeof(DevInfo)));
-  HIP_TRY(hipMemcpyAsync(hi, st.d.info, sizeof(DevInfo), hipMemcpyDeviceToHost, g_ctx.stream));
-  HIP_TRY(hipMemcpyAsync(ha, st.d.acc, sizeof(DevAccum), hipMemcpyDeviceToHost, g_ctx.stream));
+  MCR_TRY(launch_report(st, 0, false));
   HIP_TRY(hipStreamSynchronize(g_ctx.stream));
-  *info = *hi;
-  *acc = *ha;
+  *info = *st.h.info;
+  *acc = *st.h.acc;
   return MCR_OK;
 }
 
@@ -506,8 +589,7 @@ PathArgs base_args(const mcr_query* q, const Staged& st) {
 
 // Runs every path of the query once with the given loss mode.  Per-path
 // outputs (if any) are staged per chunk and copied to the caller's arrays.
-int run_paths(const mcr_query* q, const Staged& st, PathArgs a, bool per_path, bool timed,
-              float* ms) {
+int run_paths(const mcr_query* q, const Staged& st, PathArgs a, bool per_path, bool timed) {
   const uint64_t M = (uint64_t)q->paths;
   const uint64_t step = per_path ? (uint64_t)st.plan.chunk : kLaunchPaths;
   if (timed) HIP_TRY(hipEventRecord(g_ctx.ev0, g_ctx.stream));
@@ -518,19 +600,13 @@ int run_paths(const mcr_query* q, const Staged& st, PathArgs a, bool per_path, b
     a.S_out = (per_path && q->S_out) ? st.d.S_out : nullptr;
     a.loss_out = (per_path && q->loss_out) ? st.d.loss_out : nullptr;
     HIP_TRY(launch_paths(st.plan.kernel, a, g_ctx.num_cus, g_ctx.stream));
+    auto written = [] { return (int)MCR_OK; };
     if (a.S_out)
-      HIP_TRY(hipMemcpyAsync(q->S_out + s, st.d.S_out, cnt * sizeof(int32_t), hipMemcpyDeviceToHost,
-                             g_ctx.stream));
+      MCR_TRY(copy_out(st, q->S_out + s, st.d.S_out, cnt * sizeof(int32_t), written));
     if (a.loss_out)
-      HIP_TRY(hipMemcpyAsync(q->loss_out + s, st.d.loss_out, cnt * sizeof(float),
-                             hipMemcpyDeviceToHost, g_ctx.stream));
-    if (per_path) HIP_TRY(hipStreamSynchronize(g_ctx.stream));
+      MCR_TRY(copy_out(st, q->loss_out + s, st.d.loss_out, cnt * sizeof(float), written));
   }
-  if (timed) {
-    HIP_TRY(hipEventRecord(g_ctx.ev1, g_ctx.stream));
-    HIP_TRY(hipEventSynchronize(g_ctx.ev1));
-    HIP_TRY(hipEventElapsedTime(ms, g_ctx.ev0, g_ctx.ev1));
-  }
+  if (timed) HIP_TRY(hipEventRecord(g_ctx.ev1, g_ctx.stream));
   return MCR_OK;
 }
 
@@ -656,8 +732,7 @@ int refine_quantile(const mcr_query* q, const Staged& st, DevInfo info0, int al,
     a.loss_mode = kLossHist;
     a.thr_lo = 1.0f;
     a.thr_hi = 0.0f;
-    float ms = 0;
-    MCR_TRY(run_paths(q, st, a, false, false, &ms));
+    MCR_TRY(run_paths(q, st, a, false, false));
     ++*passes;
     DevAccum acc;
     DevInfo tmp;
@@ -705,7 +780,7 @@ int refine_quantile(const mcr_query* q, const Staged& st, DevInfo info0, int al,
     a.n_alpha = 1;
     a.thr_lo = 1.0f;
     a.thr_hi = 0.0f;
-    MCR_TRY(run_paths(q, st, a, false, false, &ms));
+    MCR_TRY(run_paths(q, st, a, false, false));
     ++*passes;
     MCR_TRY(read_info(st, &tmp, &acc));
     const int r = try_resolve(q, st, acc, 0, R, var, es, tail);
@@ -743,11 +818,19 @@ int run_locked(const mcr_query* q, mcr_result* r, bool noalloc) {
   a.loss_mode = (q->flags & MCR_F_VAR) ? kLossBracket : kLossNone;
   a.n_alpha = st.plan.n_alpha;
   a.s_hist = (q->flags & MCR_F_SHIST) ? st.d.s_hist : nullptr;
-  float ms = 0.0f;
-  MCR_TRY(run_paths(q, st, a, st.plan.per_path, true, &ms));
+  MCR_TRY(run_paths(q, st, a, st.plan.per_path, true));
   DevInfo info;
   DevAccum acc;
-  MCR_TRY(read_info(st, &info, &acc));
+  if (noalloc) {
+    MCR_TRY(read_info(st, &info, &acc));
+  } else {
+    MCR_TRY(launch_report(st, st.plan.n_alpha, a.s_hist != nullptr));
+    HIP_TRY(hipStreamSynchronize(g_ctx.stream));  // the one wait of a query that keeps its windows
+    info = *st.h.info;
+    acc = *st.h.acc;
+  }
+  float ms = 0.0f;
+  HIP_TRY(hipEventElapsedTime(&ms, g_ctx.ev0, g_ctx.ev1));
   MCR_TRY(check_factor(info));
 
   const int64_t M = q->paths;
@@ -762,16 +845,22 @@ int run_locked(const mcr_query* q, mcr_result* r, bool noalloc) {
 
   if (q->flags & MCR_F_SHIST) {
     const size_t nb = (size_t)q->n + 1;
-    std::vector<unsigned long long> heap(noalloc ? 0 : nb);
-    unsigned long long* h = noalloc ? g_na_shist : heap.data();
-    HIP_TRY(hipMemcpy(h, st.d.s_hist, nb * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    const unsigned long long* h = noalloc ? g_na_shist : st.h.s_hist;
+    if (noalloc)
+      HIP_TRY(hipMemcpy(g_na_shist, st.d.s_hist, nb * sizeof(unsigned long long),
+                        hipMemcpyDeviceToHost));
     for (size_t i = 0; i < nb; ++i) q->s_hist[i] = (int64_t)h[i];
   }
 
   if (q->flags & MCR_F_VAR) {
     for (int al = 0; al < st.plan.n_alpha; ++al) {
       const int64_t R = rank_of(q->alpha[al], M);
-      int res = try_resolve(q, st, acc, al, R, &r->var[al], &r->es[al], &r->tail_sum_fixed[al]);
+      int res = 1;
+      if (!noalloc && acc.gathered[al] <= st.h.cap && window_holds(M, acc, al, kGatherCap, R))
+        resolve_window(M, acc, al, st.h.win + (size_t)al * st.h.cap, R, &r->var[al], &r->es[al],
+                       &r->tail_sum_fixed[al]);
+      else
+        res = try_resolve(q, st, acc, al, R, &r->var[al], &r->es[al], &r->tail_sum_fixed[al]);
       if (res < 0) {
         set_error("copy of gathered losses failed");
         return MCR_E_DEVICE;
@@ -1494,6 +1583,7 @@ int mcr_shutdown(void) {
   HIP_TRY(hipEventDestroy(g_ctx.ev0));
   HIP_TRY(hipEventDestroy(g_ctx.ev1));
   HIP_TRY(hipEventDestroy(g_ctx.evs));
+  for (hipEvent_t e : g_ctx.evc) HIP_TRY(hipEventDestroy(e));
   destroy_forks(&g_ctx.forks);
   HIP_TRY(hipStreamDestroy(g_ctx.stream));
   g_ctx = Context();
@@ -1574,12 +1664,13 @@ int mcr_factor(int n, const double* sigma, int ld_sigma, double* L_out, mcr_fact
   MCR_TRY(ensure_init(g_ctx.device));
   HIP_TRY(hipSetDevice(g_ctx.device));
   Staged st;
-  MCR_TRY(stage_query(&q, &st, false));
+  MCR_TRY(stage_query(&q, &st, false, false, false));
+  MCR_TRY(launch_report(st, 0, false));
   DevInfo di;
-  DevAccum acc;
-  MCR_TRY(read_info(st, &di, &acc));
-  MCR_TRY(check_factor(di));
-  HIP_TRY(hipMemcpy(L_out, st.d.L, (size_t)n * n * sizeof(double), hipMemcpyDeviceToHost));
+  MCR_TRY(copy_out(st, L_out, st.d.L, (size_t)n * n * sizeof(double), [&] {
+    di = *st.h.info;
+    return check_factor(di);
+  }));
   if (info) {
     info->attempts = di.attempts;
     info->jitter = di.jitter;

@@ -621,6 +621,9 @@ hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStre
 __device__ void prep_body(const PrepArgs& a, size_t gid, size_t gsz) {
   const int n = a.n;
   const double* __restrict__ L = a.L;
+  if (a.s_hist) {
+    for (size_t e = gid; e <= (size_t)n; e += gsz) a.s_hist[e] = 0ull;
+  }
   if (a.v32) {
     for (size_t e = gid; e < (size_t)n; e += gsz) {
       a.v32[e] = (float)a.v64[e];
@@ -713,6 +716,39 @@ hipError_t launch_prep(const PrepArgs& a, hipStream_t stream) {
   if (blocks > 1024) blocks = 1024;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(k_prep, dim3(blocks), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Collect: a query's record, S histogram and window losses to pinned host memory
+// (block 0: the records; the others: kCollectBlocks per window).  One launch in
+// place of a copy each, and the windows' lengths are read where they are.
+// ---------------------------------------------------------------------------
+constexpr int kCollectBlocks = 16;
+
+__global__ __launch_bounds__(256) void k_collect(CollectArgs a) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0) {
+    auto copy = [&](void* dst, const void* src, size_t bytes) {
+      for (size_t i = tid; i < bytes / 4; i += 256)
+        static_cast<uint32_t*>(dst)[i] = static_cast<const uint32_t*>(src)[i];
+    };
+    static_assert(sizeof(DevInfo) % 4 == 0 && sizeof(DevAccum) % 4 == 0, "copied as words");
+    copy(a.h_info, a.info, sizeof(DevInfo));
+    copy(a.h_acc, a.acc, sizeof(DevAccum));
+    if (a.s_hist) copy(a.h_hist, a.s_hist, (size_t)(a.n + 1) * sizeof(unsigned long long));
+    return;
+  }
+  const int al = (blockIdx.x - 1) / kCollectBlocks, part = (blockIdx.x - 1) % kCollectBlocks;
+  const unsigned long long g = a.acc->gathered[al];
+  const unsigned lim = a.cap < a.gather_cap ? a.cap : a.gather_cap;
+  const unsigned cnt = g < lim ? (unsigned)g : lim;
+  for (unsigned i = part * 256 + tid; i < cnt; i += kCollectBlocks * 256)
+    a.h_win[(size_t)al * a.cap + i] = a.gather[(size_t)al * a.gather_cap + i];
+}
+
+hipError_t launch_collect(const CollectArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL(k_collect, dim3(1 + kCollectBlocks * a.n_alpha), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

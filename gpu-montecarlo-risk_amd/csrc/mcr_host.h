@@ -65,6 +65,7 @@ struct Context {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evs = nullptr;  // start of a query's device work (after its uploads)
+  hipEvent_t evc[2] = {};    // the two staging buffers of copy_out
   void* arena = nullptr;
   size_t arena_bytes = 0;
   void* host = nullptr;  // pinned staging

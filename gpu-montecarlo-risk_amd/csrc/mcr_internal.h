@@ -125,11 +125,29 @@ struct PrepArgs {
   float* v32;
   uint4* lfrag;
   float* rowinit;
+  unsigned long long* s_hist;  // optional [n+1]: cleared
+};
+
+// What a query reports, written to pinned host memory by one kernel behind its
+// path kernels.
+struct CollectArgs {
+  const DevInfo* info;
+  const DevAccum* acc;
+  const float* gather;              // [n_alpha][gather_cap]
+  const unsigned long long* s_hist; // optional [n+1]
+  unsigned gather_cap;
+  int n, n_alpha;
+  unsigned cap;                     // losses copied per window, at most
+  DevInfo* h_info;
+  DevAccum* h_acc;
+  float* h_win;                     // [n_alpha][cap]
+  unsigned long long* h_hist;
 };
 
 // Launchers (mcr_device.hip).  All asynchronous on `stream`.
 hipError_t launch_factor(const FactorArgs& a, hipStream_t stream);
 hipError_t launch_prep(const PrepArgs& a, hipStream_t stream);
+hipError_t launch_collect(const CollectArgs& a, hipStream_t stream);
 hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStream_t stream);
 hipError_t launch_prep_batch(const PrepArgs* pas, int nq, int max_n, hipStream_t stream);
 

@@ -319,3 +319,18 @@ def test_subrange_of_large_run_matches_oracle(mcr, orc):
     99,980,000 of the n = 50 workload equals the oracle's same window."""
     _exact_case(mcr, orc, 50, 20000, 10, mcr.KERNEL_VALU_REG, seed=7, path_offset=99_980_000, K=5,
                 msd=952)
+
+
+@pytest.mark.parametrize("paths", [262143, 262144, 262145, 524288, 786433])
+def test_per_path_outputs_across_staging_pieces(mcr, paths):
+    """S and loss of paths on both sides of the 1 MiB staging pieces' edges: the
+    parts of a run split elsewhere, the crash count and the S histogram."""
+    mu, sigma = factor_like(7, 2, 91, T=1500)
+    r = mcr.run(mu, sigma, 0.02, 2, paths, 5, want_S=True, want_loss=True, want_hist=True)
+    cut = 100_003
+    a = mcr.run(mu, sigma, 0.02, 2, cut, 5, want_S=True, want_loss=True)
+    b = mcr.run(mu, sigma, 0.02, 2, paths - cut, 5, want_S=True, want_loss=True, path_offset=cut)
+    assert np.array_equal(r.S, np.concatenate([a.S, b.S]))
+    assert np.array_equal(r.loss, np.concatenate([a.loss, b.loss]))
+    assert np.array_equal(r.s_hist, np.bincount(r.S, minlength=8))
+    assert r.count == int((r.S >= 2).sum())
