@@ -26,7 +26,7 @@ namespace mcr {
 // and with no overlap to gain there is nothing to interleave: one barrier per
 // chunk.  Tiles go to the four SIMDs largest first, to the least loaded one.
 // Per 1e6 paths, this kernel against the vector kernels it replaced (tile to n =
-// 608, column chunks past it): n = 143 0.37 / 0.56 ms, n = 300 1.09 / 2.15, n =
+// 608, column chunks past it): n = 143 0.35 / 0.56 ms, n = 300 1.03 / 2.15, n =
 // 600 3.5 / 6.5, n = 1024 10.3 / 23.7; n = 600 is 103 TFLOP/s of n (n + 1) per
 // path, two thirds of the matrix rate with the normals' time and the padded
 // halves of the diagonal tiles in it.
@@ -259,19 +259,25 @@ __global__ __launch_bounds__(64 * NW, 4) void k_f32_lds(PathArgs a) {
   }
 }
 
-// Waves per workgroup and workgroups per CU.  The normals of 64 paths take n / 4
-// KiB, so at large n one workgroup fills a CU's LDS: it then has 16 waves, 8
-// where two or three fit, else 4 (each wave has two tile slots, T <= 2 NW in
-// every case: n <= 148 for 4 waves, n <= 308 for 8).
+// Waves per workgroup and workgroups per CU, four waves per SIMD in all.  The
+// normals of 64 paths take n / 4 KiB, so at large n one workgroup fills a CU's LDS
+// and has 16 waves; 8 where two fit (n <= 304), 4 where four do (n <= 152), so
+// that one's normals run beside another's products and fewer waves meet at a
+// barrier: 4e11 / (n^2 + 40 n) paths on 4 against 8 waves n = 143 5.29 / 5.71 ms,
+// n = 150 5.00 / 5.50; on 8 against 16 n = 301 4.02 / 4.24.  Two tile slots per
+// wave cover T in every case.
 F32Shape f32_shape(int n) {
   F32Shape s;
   const int S = (n + 7) / 8;
   s.lds = (size_t)(n <= kMaxN ? S : kChunkCols / 8) * 128 * sizeof(float4) +
           ((n + 1) * sizeof(unsigned) + 15) / 16 * 16;
-  const size_t stat = sizeof(int) * 16 * 64 + sizeof(float) * 64 + sizeof(LdsTally);
-  s.per_cu = std::max(1, std::min(4, (int)((160 * 1024) / (s.lds + stat))));
-  s.waves = s.per_cu == 1 ? 16 : (s.per_cu <= 3 ? 8 : 4);
-  if (s.waves == 8) s.per_cu = 2;  // four waves per SIMD
+  // static LDS: counts and losses of 64 paths per wave, the tally
+  auto fits = [&](int waves) {
+    const size_t stat = sizeof(int) * waves * 64 + sizeof(float) * 64 + sizeof(LdsTally);
+    return (int)((160 * 1024) / (s.lds + stat));
+  };
+  s.waves = fits(4) >= 4 ? 4 : (fits(8) >= 2 ? 8 : 16);
+  s.per_cu = 16 / s.waves;  // four waves per SIMD
   s.kernel = s.waves == 16 ? k_f32_lds<16> : (s.waves == 8 ? k_f32_lds<8> : k_f32_lds<4>);
   return s;
 }

@@ -188,6 +188,13 @@ def test_lds_kernel_exact_at_shape_edges(mcr, orc, n, kernel):
     _exact_case(mcr, orc, n, 1500, max(1, n // 5), kernel, path_offset=2**32 - 741)
 
 
+@pytest.mark.parametrize("n", [152, 153, 304, 305])
+def test_lds_kernel_exact_where_workgroups_fit(mcr, orc, n):
+    """The same at the last n where four workgroups (of four waves) and two (of
+    eight) share a compute unit's LDS, and the first where they do not."""
+    _exact_case(mcr, orc, n, 1500, max(1, n // 5), 2, path_offset=2**32 - 741)
+
+
 @pytest.mark.parametrize("n", [1, 5, 9, 50, 129, 257, 600, 608, 609, 700, 1000, 1024])
 def test_chunk_kernel_exact(mcr, orc, n):
     """The column-chunk kernel (any n <= 1024; fp32 past 608): per-path
