@@ -336,8 +336,10 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
   const bool diag = lane < 32;
   const int row = diag ? k0 + r : k0 + kBlk * (1 + 4 * blk + wave) + r;
   const bool valid = row < n;
-  const double* __restrict__ src = s <= 1 ? a.A : a.L;
   double* __restrict__ L = a.L;
+  // the diagonal block, which one wave finishes while others may still have to
+  // read it, waits in the zero triangle (see chol_update)
+  const double* __restrict__ src = s <= 1 ? a.A : diag ? L - (size_t)kBlk * n : L;
   double x[kBlk];
 #pragma unroll
   for (int c = 0; c < kBlk; ++c)
@@ -414,7 +416,10 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
   }
 }
 
-// The tile at (r0, c0) of the lower triangle takes block column kp's update.
+// The tile at (r0, c0) of the lower triangle takes block column s - 1's update.
+// The next launch's diagonal block goes to the rows 32 above its place, in the
+// zero triangle: that launch's workgroups all read it, at any time while the
+// first of them writes the factored block to L.  chol_clear zeroes it again.
 __device__ void chol_update(const FactorArgs& a, int s, int r0, int c0, CholShared& sh) {
   const int n = a.n, kp = kBlk * (s - 1);
   const double* __restrict__ src = s == 1 ? a.A : a.L;
@@ -459,8 +464,19 @@ __device__ void chol_update(const FactorArgs& a, int s, int r0, int c0, CholShar
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int i = r0 + ri + u, j = c0 + cj + v;
-      if (i < n && j <= i) L[(size_t)i * n + j] = x[u][v];
+      if (i < n && j <= i) {
+        const int up = i < kBlk * (s + 2) ? kBlk : 0;
+        L[(size_t)(i - up) * n + j] = x[u][v];
+      }
     }
+}
+
+// The place above the diagonal where block s waited (s >= 2).
+__device__ void chol_clear(const FactorArgs& a, int s) {
+  for (int e = threadIdx.x; e < kBlk * kBlk; e += blockDim.x) {
+    const int j = kBlk * s + e % kBlk;
+    if (j < a.n) a.L[(size_t)(kBlk * (s - 1) + e / kBlk) * a.n + j] = 0.0;
+  }
 }
 
 // Launch 0 beside the first panel: the zero upper triangle of L, and the search
@@ -511,6 +527,7 @@ __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
   if ((int)blockIdx.x == np) {
     const int j = kBlk * (s - 1) + threadIdx.x;
     if (threadIdx.x < kBlk) a.v64[j] = loading_of(a, j);
+    if (s > 2) chol_clear(a, s - 1);
     return;
   }
   const int t = blockIdx.x - np - 1;
@@ -566,7 +583,9 @@ __device__ void factor_finish(const FactorArgs& a, FactorShared<MAXN>& sh) {
     __syncthreads();  // the record is read before anyone writes it
     if (!cholesky_body(a, sh, &attempts, &clamped, &last_fail, &delta)) return;
   } else {
-    j0 = kBlk * ((a.n - 1) / kBlk);  // the launches left the last block column
+    const int last = (a.n - 1) / kBlk;  // the launches left this block column's loading
+    j0 = kBlk * last;
+    if (last > 1) chol_clear(a, last);
   }
   if (a.finfo && !a.reuse && tid == 0) {
     a.finfo->attempts = attempts;
