@@ -291,23 +291,27 @@ __device__ void moments_body(const FactorArgs& a, double* red, int j0, int attem
 // First attempt, launch s of ceil(n / 32): block column s (columns 32s .. 32s +
 // 31) is finished and the columns right of it take the update of block column
 // s - 1, which only needs what launch s - 1 left behind:
-//   panel waves   rows 0-31 of the wave's 64 are the diagonal block (every wave
-//                 factors it for itself: no exchange, no barrier), rows 32-63 its
-//                 own 32 rows below.  A lane holds its row's 32 entries, takes
-//                 block column s - 1's update and then the 32 columns, the
+//   panels        a workgroup per 32 rows below the diagonal block, which each
+//                 factors for itself: 64 rows come in coalesced and take block
+//                 column s - 1's update on v_mfma_f64_16x16x4, then 16 columns
+//                 at a time go through the first wave, a row per lane, the
 //                 pivots and the diagonal block's entries coming by readlane.
-//   update tiles  64 x 64, block column s - 1's product subtracted;
+//   update tiles  64 x 64, block column s - 1's product subtracted (same
+//                 instruction);
 //   loading       block column s - 1's part of v = L^T w, a column per lane.
 // Every entry sees the operations of a right-looking factorisation by panels of
 // 16 columns in its order (per panel a chain of 16 fused multiply-adds from zero,
 // then one subtraction; inside a panel one fused multiply-add per column), so L
 // has the bits that cholesky_body's algorithm gives it.
-// Bound: the chain of 32 square roots and reciprocals of a launch (about 8 of its
-// 21 us; its loads and stores cross the XCDs' caches).  Factor and layouts at n =
-// 50 / 143 / 301 / 600 / 1024: 52 / 133 / 263 / 414 / 773 us; one workgroup did the
-// whole of it before in 67 / 163 / 460 / 1809 / 6768.
+// Bound: the chain of 32 square roots and reciprocals of a launch (4.3 of its 11
+// us at n = 600), then the latency of its loads.  All launches, n = 15 / 143 /
+// 301 / 600 / 1024: 14 / 55 / 107 / 213 / 434 us; with a row per lane in global
+// memory too (64 lines to a load) and the update on the vector unit, its operands
+// broadcast from LDS, 20 / 114 / 251 / 413 / 775; on one workgroup 1809 us at n =
+// 600, 6768 at n = 1024.
 // ---------------------------------------------------------------------------
 constexpr int kBlk = 32;
+constexpr int kLoadRows = 128;  // rows of L^T w in LDS at a time
 
 // double of lane `src` (a constant) in every lane
 __device__ __forceinline__ double bcast(double v, int src) {
@@ -317,100 +321,121 @@ __device__ __forceinline__ double bcast(double v, int src) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
 struct CholShared {
   union {
     struct {
-      double prev[kBlk][kBlk];       // L[diagonal block's rows][block column s - 1]
-      double cross[4][kPanel][kPanel];  // per wave: rows 16-31 of the diagonal block, first panel
+      double prev[64][33];  // block column s - 1 in the panel's rows
+      double x[64][34];     // block column s there
     } p;
     struct {
-      double a[kBlk][68], b[kBlk][68];  // [column of s - 1][row of the tile]
+      double a[64][33], b[64][33];  // block column s - 1 in the tile's rows and columns
     } u;
+    double prod[kLoadRows][kBlk];  // L_ij w_i
   };
   int failed;
 } __attribute__((aligned(16)));
 
+// 16 x 16 products of rows ra .. and rb .. over 16 columns from p: a chain of 16
+// fused multiply-adds from zero per entry, p ascending (the instruction fuses
+// and takes its four products in that order).  Entry i of lane l: row
+// 4 i + l / 16, column l % 16.
+template <int LD>
+__device__ __forceinline__ f64x4 chain16(const double (&va)[64][LD], int ra,
+                                         const double (&vb)[64][LD], int rb, int p) {
+  const int lane = threadIdx.x & 63, m = lane & 15, k = lane >> 4;
+  f64x4 acc = {};
+#pragma unroll
+  for (int q = 0; q < 16; q += 4)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(va[ra + m][p + q + k], vb[rb + m][p + q + k], acc, 0, 0, 0);
+  return acc;
+}
+
+// Columns q .. q + 15 of the panel, a row per lane (rows 0-31 the diagonal
+// block's): x the row's entries, piv the pivot of the lane's column as found.
+__device__ __forceinline__ void chol_columns(double (&x)[kPanel], int q, double* piv) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int c = 0; c < kPanel; ++c) {
+    const double d = bcast(x[c], q + c);
+    if (lane == q + c) *piv = d;
+    const double ljj = sqrt(d), rl = 1.0 / ljj;
+    const double lr = x[c] * rl;
+    x[c] = lane == q + c ? ljj : lr;
+#pragma unroll
+    for (int c2 = c + 1; c2 < kPanel; ++c2) x[c2] = fma(-lr, bcast(lr, q + c2), x[c2]);
+  }
+}
+
 __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) {
   const int n = a.n, k0 = kBlk * s, kb = min(kBlk, n - k0);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31;
-  const bool diag = lane < 32;
-  const int row = diag ? k0 + r : k0 + kBlk * (1 + 4 * blk + wave) + r;
-  const bool valid = row < n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double* __restrict__ L = a.L;
-  // the diagonal block, which one wave finishes while others may still have to
-  // read it, waits in the zero triangle (see chol_update)
+  // row t of the panel: the diagonal block's, then the workgroup's own
+  auto row_of = [&](int t) { return t < kBlk ? k0 + t : k0 + kBlk * blk + t; };
+
+  // entry i of half h: row 16 wave + 4 i + lane / 16, column 16 h + lane % 16
+  f64x4 x[2];
+  const bool diag = wave < 2;
+  // the diagonal block, which one workgroup finishes while others may still have
+  // to read it, waits in the zero triangle (see chol_update)
   const double* __restrict__ src = s <= 1 ? a.A : diag ? L - (size_t)kBlk * n : L;
-  double x[kBlk];
 #pragma unroll
-  for (int c = 0; c < kBlk; ++c)
-    x[c] = valid && c < kb && (!diag || c <= r) ? src[(size_t)row * n + k0 + c]
-                                                : (diag && c == r ? 1.0 : 0.0);  // identity pads
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * wave + 4 * i + (lane >> 4), c = 16 * h + (lane & 15), row = row_of(t);
+      x[h][i] = row < n && c < kb && (!diag || c <= t) ? src[(size_t)row * n + k0 + c]
+                                                       : (diag && c == t ? 1.0 : 0.0);  // identity pads
+    }
   if (s > 0) {
-    const int kp = k0 - kBlk;
-    for (int e = threadIdx.x; e < kBlk * kBlk; e += blockDim.x) {
-      const int j = e / kBlk, p = e % kBlk;
-      sh.p.prev[j][p] = k0 + j < n ? L[(size_t)(k0 + j) * n + kp + p] : 0.0;
-    }
-    double lp[kBlk];
+    double l[64 * kBlk / 256];
 #pragma unroll
-    for (int p = 0; p < kBlk; ++p) lp[p] = valid ? L[(size_t)row * n + kp + p] : 0.0;
+    for (int u = 0; u < 64 * kBlk / 256; ++u) {
+      const int t = 8 * u + threadIdx.x / kBlk, row = row_of(t);
+      l[u] = row < n ? L[(size_t)row * n + k0 - kBlk + threadIdx.x % kBlk] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 64 * kBlk / 256; ++u)
+      sh.p.prev[8 * u + threadIdx.x / kBlk][threadIdx.x % kBlk] = l[u];
     __syncthreads();
-    // four columns at a time: eight independent chains keep the unit busy
 #pragma unroll
-    for (int j = 0; j < kBlk; j += 4) {
-      double acc[4][2] = {};
+    for (int p = 0; p < kBlk; p += kPanel)
 #pragma unroll
-      for (int p = 0; p < kPanel; ++p)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          acc[u][0] = fma(lp[p], sh.p.prev[j + u][p], acc[u][0]);
-          acc[u][1] = fma(lp[kPanel + p], sh.p.prev[j + u][kPanel + p], acc[u][1]);
-        }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) x[j + u] = x[j + u] - acc[u][0] - acc[u][1];
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      for (int h = 0; h < 2; ++h) x[h] -= chain16(sh.p.prev, 16 * wave, sh.p.prev, 16 * h, p);
   }
-  double piv = 0.0;  // this lane's pivot, as its column found it
+  // 16 columns at a time: into LDS, through the first wave's registers and back
+  double piv = 0.0;
 #pragma unroll
-  for (int q = 0; q < kBlk; q += kPanel) {
+  for (int h = 0; h < 2; ++h) {
+    if (kPanel * h >= kb) break;
+    if (h > 0) x[h] -= chain16(sh.p.x, 16 * wave, sh.p.x, kPanel, 0);
 #pragma unroll
-    for (int c = q; c < q + kPanel; ++c) {
-      const double d = bcast(x[c], c);
-      if (lane == c) piv = d;
-      const double ljj = sqrt(d), rl = 1.0 / ljj;
-      const double lr = x[c] * rl;
-      x[c] = lane == c ? ljj : lr;
+    for (int i = 0; i < 4; ++i)
+      sh.p.x[16 * wave + 4 * i + (lane >> 4)][kPanel * h + (lane & 15)] = x[h][i];
+    __syncthreads();
+    if (wave == 0) {
+      double y[kPanel];
 #pragma unroll
-      for (int c2 = c + 1; c2 < q + kPanel; ++c2) x[c2] = fma(-lr, bcast(lr, c2), x[c2]);
+      for (int c = 0; c < kPanel; ++c) y[c] = sh.p.x[lane][kPanel * h + c];
+      chol_columns(y, kPanel * h, &piv);
+#pragma unroll
+      for (int c = 0; c < kPanel; ++c) sh.p.x[lane][kPanel * h + c] = y[c];
     }
-    if (q == 0) {
-      // the first panel's update of the second's columns
-      if (diag && r >= kPanel) {
-#pragma unroll
-        for (int p = 0; p < kPanel; ++p) sh.p.cross[wave][r - kPanel][p] = x[p];
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int c = 0; c < kPanel; ++c) {
-        double acc = 0.0;
-#pragma unroll
-        for (int p = 0; p < kPanel; ++p) acc = fma(x[p], sh.p.cross[wave][c][p], acc);
-        x[kPanel + c] -= acc;
-      }
-    }
+    __syncthreads();
   }
-  const bool first = blk == 0 && wave == 0;
-  if (valid && (!diag || first)) {
 #pragma unroll
-    for (int c = 0; c < kBlk; ++c)
-      if (c < kb) L[(size_t)row * n + k0 + c] = diag && c > r ? 0.0 : x[c];
+  for (int u = 0; u < 64 * kBlk / 256; ++u) {
+    const int t = 8 * u + threadIdx.x / kBlk, c = threadIdx.x % kBlk, row = row_of(t);
+    if (row < n && c < kb && (t >= kBlk || blk == 0))
+      L[(size_t)row * n + k0 + c] = c > t ? 0.0 : sh.p.x[t][c];
   }
-  if (first) {
-    const double ajj = diag && valid ? a.A[(size_t)row * n + row] : 1.0;
+  if (blk == 0 && wave == 0) {
+    const bool col = lane < kb;
+    const double ajj = col ? a.A[(size_t)(k0 + lane) * n + k0 + lane] : 1.0;
     const double tol = (double)n * DBL_EPSILON * ajj;
-    const unsigned long long bad = __ballot(diag && r < kb && (!(piv > tol) || !isfinite(piv)));
+    const unsigned long long bad = __ballot(col && (!(piv > tol) || !isfinite(piv)));
     const int fail = bad ? k0 + __ffsll((long long)bad) : 0;  // first failing column + 1
     if (lane == 0 && (s == 0 || fail)) a.info->fail_col = fail;
   }
@@ -422,53 +447,86 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
 // first of them writes the factored block to L.  chol_clear zeroes it again.
 __device__ void chol_update(const FactorArgs& a, int s, int r0, int c0, CholShared& sh) {
   const int n = a.n, kp = kBlk * (s - 1);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const double* __restrict__ src = s == 1 ? a.A : a.L;
   double* __restrict__ L = a.L;
-  for (int e = threadIdx.x; e < 64 * kBlk; e += blockDim.x) {
-    const int i = e / kBlk, p = e % kBlk;
-    sh.u.a[p][i] = r0 + i < n ? L[(size_t)(r0 + i) * n + kp + p] : 0.0;
-    sh.u.b[p][i] = c0 + i < n ? L[(size_t)(c0 + i) * n + kp + p] : 0.0;
+  double la[64 * kBlk / 256], lb[64 * kBlk / 256];
+#pragma unroll
+  for (int u = 0; u < 64 * kBlk / 256; ++u) {
+    const int i = 8 * u + threadIdx.x / kBlk, p = threadIdx.x % kBlk;
+    la[u] = r0 + i < n ? L[(size_t)(r0 + i) * n + kp + p] : 0.0;
+    lb[u] = c0 + i < n ? L[(size_t)(c0 + i) * n + kp + p] : 0.0;
   }
-  const int ri = 4 * (threadIdx.x >> 4), cj = 4 * (threadIdx.x & 15);
-  double x[4][4];
+  // a wave's 16 rows: entry i of tile v: row 4 i + lane / 16, column 16 v + lane % 16
+  const int i0 = r0 + 16 * wave + (lane >> 4), j0 = c0 + (lane & 15);
+  f64x4 x[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+  for (int v = 0; v < 4; ++v)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = r0 + ri + u, j = c0 + cj + v;
-      x[u][v] = i < n && j <= i ? src[(size_t)i * n + j] : 0.0;
-    }
+    for (int i = 0; i < 4; ++i)
+      x[v][i] = i0 + 4 * i < n && j0 + 16 * v <= i0 + 4 * i ? src[(size_t)(i0 + 4 * i) * n + j0 + 16 * v] : 0.0;
+#pragma unroll
+  for (int u = 0; u < 64 * kBlk / 256; ++u) {
+    const int i = 8 * u + threadIdx.x / kBlk, p = threadIdx.x % kBlk;
+    sh.u.a[i][p] = la[u];
+    sh.u.b[i][p] = lb[u];
+  }
   __syncthreads();
 #pragma unroll
-  for (int h = 0; h < kBlk; h += kPanel) {
-    double acc[4][4] = {};
-#pragma unroll 4
-    for (int p = h; p < h + kPanel; ++p) {
-      const double2* pa = (const double2*)&sh.u.a[p][ri];
-      const double2* pb = (const double2*)&sh.u.b[p][cj];
-      const double2 a01 = pa[0], a23 = pa[1], b01 = pb[0], b23 = pb[1];
-      const double av[4] = {a01.x, a01.y, a23.x, a23.y};
-      const double bv[4] = {b01.x, b01.y, b23.x, b23.y};
+  for (int h = 0; h < kBlk; h += kPanel)
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+    for (int v = 0; v < 4; ++v) x[v] -= chain16(sh.u.a, 16 * wave, sh.u.b, 16 * v, h);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = fma(av[u], bv[v], acc[u][v]);
-    }
+  for (int v = 0; v < 4; ++v)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x[u][v] -= acc[u][v];
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = r0 + ri + u, j = c0 + cj + v;
-      if (i < n && j <= i) {
-        const int up = i < kBlk * (s + 2) ? kBlk : 0;
-        L[(size_t)(i - up) * n + j] = x[u][v];
+    for (int i = 0; i < 4; ++i) {
+      const int r = i0 + 4 * i, j = j0 + 16 * v;
+      if (r < n && j <= r) {
+        const int up = r < kBlk * (s + 2) ? kBlk : 0;
+        L[(size_t)(r - up) * n + j] = x[v][i];
       }
     }
+}
+
+// v_j of block column s - 1 (loading_of's sum): the workgroup loads and
+// multiplies kLoadRows rows at a time, the next ones on their way, and a lane per
+// column adds them up.
+__device__ void chol_loading(const FactorArgs& a, int s, CholShared& sh) {
+  const int n = a.n, c = threadIdx.x % kBlk, k0 = kBlk * (s - 1);
+  const double* __restrict__ col = a.L + k0 + c;
+  constexpr int kPer = kLoadRows * kBlk / 256;
+  double l[kPer], w[kPer], sum = 0.0;
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int i = i0 + 8 * u + threadIdx.x / kBlk;
+      const bool on = i < n && i >= k0 + c;
+      l[u] = on ? col[(size_t)i * n] : 0.0;
+      w[u] = on ? a.w[i] : 0.0;
+    }
+  };
+  load(k0);
+  for (int i0 = k0; i0 < n; i0 += kLoadRows) {
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) sh.prod[8 * u + threadIdx.x / kBlk][c] = l[u] * w[u];
+    __syncthreads();
+    load(i0 + kLoadRows);
+    if (threadIdx.x < kBlk) {
+      // rows above the diagonal are zeros here, and adding one changes nothing
+      const int m = min(kLoadRows, n - i0);
+      int i = 0;
+      for (; i + 16 <= m; i += 16) {
+        double p[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) p[u] = sh.prod[i + u][c];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) sum += p[u];
+      }
+      for (; i < m; ++i) sum += sh.prod[i][c];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < kBlk) a.v64[k0 + c] = sum;
 }
 
 // The place above the diagonal where block s waited (s >= 2).
@@ -497,8 +555,8 @@ __device__ void chol_upper(const FactorArgs& a, int r0, int c0) {
 }
 
 __host__ __device__ inline int chol_panel_wgs(int n, int s) {
-  const int below = n - kBlk * (s + 1);  // rows under the diagonal block, 128 per workgroup
-  return below > 0 ? (below + 127) / 128 : 1;
+  const int below = n - kBlk * (s + 1);  // rows under the diagonal block
+  return below > 0 ? (below + kBlk - 1) / kBlk : 1;
 }
 __host__ __device__ inline int chol_step_wgs(int n, int s) {
   if (kBlk * s >= n) return 0;
@@ -525,8 +583,7 @@ __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
     return;
   }
   if ((int)blockIdx.x == np) {
-    const int j = kBlk * (s - 1) + threadIdx.x;
-    if (threadIdx.x < kBlk) a.v64[j] = loading_of(a, j);
+    chol_loading(a, s, sh);
     if (s > 2) chol_clear(a, s - 1);
     return;
   }
