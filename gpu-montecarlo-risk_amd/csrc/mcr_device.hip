@@ -303,9 +303,9 @@ __device__ void moments_body(const FactorArgs& a, double* red, int j0, int attem
 // 16 columns in its order (per panel a chain of 16 fused multiply-adds from zero,
 // then one subtraction; inside a panel one fused multiply-add per column), so L
 // has the bits that cholesky_body's algorithm gives it.
-// Bound: the chain of 32 square roots and reciprocals of a launch (4.3 of its 11
+// Bound: the chain of 32 square roots and reciprocals of a launch (3.7 of its 10
 // us at n = 600), then the latency of its loads.  All launches, n = 15 / 143 /
-// 301 / 600 / 1024: 14 / 55 / 107 / 213 / 434 us; with a row per lane in global
+// 301 / 600 / 1024: 13 / 47 / 92 / 194 / 414 us; with a row per lane in global
 // memory too (64 lines to a load) and the update on the vector unit, its operands
 // broadcast from LDS, 20 / 114 / 251 / 413 / 775; on one workgroup 1809 us at n =
 // 600, 6768 at n = 1024.
@@ -352,9 +352,68 @@ __device__ __forceinline__ f64x4 chain16(const double (&va)[64][LD], int ra,
   return acc;
 }
 
+// sqrt(d) and its correctly rounded reciprocal in kStages steps (all with one
+// use of the vector unit's latency), without the library's care for the ends of
+// the range: d in [2^-752, 2^1000].  Goldschmidt's coupled iteration for the
+// root and half its reciprocal from the hardware's estimate, then Markstein's
+// correction of each by its fused residual ("Computation of elementary functions
+// on the IBM RISC System/6000 processor", 1990); the reciprocal starts from the
+// root's instead of an estimate of its own.  The same bits as sqrt(d) and 1.0 /
+// sqrt(d) over 2e8 random, square and near-square d, but for the reciprocal of a
+// root whose significand is all ones (d the last double below a power of four),
+// one unit in the last place off.
+struct RootRecip {
+  double d, g, h, q, e;
+  static constexpr int kStages = 10;
+  __device__ __forceinline__ void stage(int k) {
+    if (k == 0) h = __builtin_amdgcn_rsq(d);
+    if (k == 1) g = d * h, h = 0.5 * h;
+    if (k == 2) e = fma(-h, g, 0.5);
+    if (k == 3) g = fma(g, e, g), h = fma(h, e, h);
+    if (k == 4) e = fma(-g, g, d), q = h + h;
+    if (k == 5) g = fma(e, h, g);
+    if (k == 6) e = fma(-g, g, d), d = fma(-g, q, 1.0);
+    if (k == 7) g = fma(e, h, g), q = fma(d, q, q);
+    if (k == 8) e = fma(-g, q, 1.0);
+    if (k == 9) q = fma(e, q, q);
+  }
+};
+
 // Columns q .. q + 15 of the panel, a row per lane (rows 0-31 the diagonal
 // block's): x the row's entries, piv the pivot of the lane's column as found.
+// One wave runs this alone, so instruction order is what hides latency: the next
+// column takes its update first, and a step of its root stands before each of
+// the other columns' updates.  All launches, n = 143 / 301 / 600: 47 / 92 / 194
+// us; a column after the other 50 / 98 / 201, with the library's root and
+// reciprocal 55 / 107 / 213.
 __device__ __forceinline__ void chol_columns(double (&x)[kPanel], int q, double* piv) {
+  const int lane = threadIdx.x & 63;
+  RootRecip rt;
+  rt.d = bcast(x[0], q);
+  if (lane == q) *piv = rt.d;
+#pragma unroll
+  for (int k = 0; k < RootRecip::kStages; ++k) rt.stage(k);
+#pragma unroll
+  for (int c = 0; c < kPanel; ++c) {
+    const double lr = x[c] * rt.q;
+    x[c] = lane == q + c ? rt.g : lr;
+    if (c + 1 == kPanel) break;
+    x[c + 1] = fma(-lr, bcast(lr, q + c + 1), x[c + 1]);
+    rt.d = bcast(x[c + 1], q + c + 1);
+    if (lane == q + c + 1) *piv = rt.d;
+#pragma unroll
+    for (int k = 0; k < RootRecip::kStages; ++k) {
+      rt.stage(k);
+      const int c2 = c + 2 + k;
+      if (c2 < kPanel) x[c2] = fma(-lr, bcast(lr, q + c2), x[c2]);
+    }
+#pragma unroll
+    for (int c2 = c + 2 + RootRecip::kStages; c2 < kPanel; ++c2) x[c2] = fma(-lr, bcast(lr, q + c2), x[c2]);
+  }
+}
+
+// The same with the library's root and reciprocal, for pivots of any size.
+__device__ __forceinline__ void chol_columns_any(double (&x)[kPanel], int q, double* piv) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int c = 0; c < kPanel; ++c) {
@@ -405,6 +464,11 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
 #pragma unroll
       for (int h = 0; h < 2; ++h) x[h] -= chain16(sh.p.prev, 16 * wave, sh.p.prev, 16 * h, p);
   }
+  // the block's diagonal of A: its pivots are no larger, and none is smaller than
+  // n eps of its own but one that fails
+  const bool col = lane < kb;
+  const double ajj = col ? a.A[(size_t)(k0 + lane) * n + k0 + lane] : 1.0;
+  const bool mid = __ballot(!(ajj > 0x1p-700 && ajj < 0x1p+990)) == 0ull;
   // 16 columns at a time: into LDS, through the first wave's registers and back
   double piv = 0.0;
 #pragma unroll
@@ -419,7 +483,10 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
       double y[kPanel];
 #pragma unroll
       for (int c = 0; c < kPanel; ++c) y[c] = sh.p.x[lane][kPanel * h + c];
-      chol_columns(y, kPanel * h, &piv);
+      if (mid)
+        chol_columns(y, kPanel * h, &piv);
+      else
+        chol_columns_any(y, kPanel * h, &piv);
 #pragma unroll
       for (int c = 0; c < kPanel; ++c) sh.p.x[lane][kPanel * h + c] = y[c];
     }
@@ -432,8 +499,6 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
       L[(size_t)row * n + k0 + c] = c > t ? 0.0 : sh.p.x[t][c];
   }
   if (blk == 0 && wave == 0) {
-    const bool col = lane < kb;
-    const double ajj = col ? a.A[(size_t)(k0 + lane) * n + k0 + lane] : 1.0;
     const double tol = (double)n * DBL_EPSILON * ajj;
     const unsigned long long bad = __ballot(col && (!(piv > tol) || !isfinite(piv)));
     const int fail = bad ? k0 + __ffsll((long long)bad) : 0;  // first failing column + 1

@@ -110,6 +110,19 @@ def test_factor_retries_from_any_column(mcr, orc, col):
         assert e.value.code == mcr.MCR_E_FACTOR
 
 
+@pytest.mark.parametrize("exp", [-760, -702, -698, 0, 988, 992, 1010])
+@pytest.mark.parametrize("n", [7, 16, 70])
+def test_factor_scales_with_the_covariance(mcr, n, exp):
+    """A covariance times 4^k has the factor times 2^k, bit for bit, on either
+    side of the diagonal sizes that the short root and reciprocal take."""
+    A = random_spd(n, 300 + n, cond=50.0)
+    A /= np.max(np.diag(A))
+    L0 = mcr.factor(A)[0]
+    L, att, jit, cl = mcr.factor(np.ldexp(A, exp))
+    assert (att, jit, cl) == (1, 0.0, 0)
+    assert np.array_equal(L, np.ldexp(L0, exp // 2))
+
+
 def test_factor_clamp_fallback(mcr, orc):
     A = np.diag([1.0, 1.0, -0.5, 1.0]) * 1e-4
     L, att, jit, cl = mcr.factor(A)
