@@ -298,14 +298,14 @@ __device__ void moments_body(const FactorArgs& a, double* red, int j0, int attem
 //                 pivots and the diagonal block's entries coming by readlane.
 //   update tiles  64 x 64, block column s - 1's product subtracted (same
 //                 instruction);
-//   loading       block column s - 1's part of v = L^T w, a column per lane.
+//   loading       pieces of v = L^T w, a column per lane (see chol_loading).
 // Every entry sees the operations of a right-looking factorisation by panels of
 // 16 columns in its order (per panel a chain of 16 fused multiply-adds from zero,
 // then one subtraction; inside a panel one fused multiply-add per column), so L
 // has the bits that cholesky_body's algorithm gives it.
 // Bound: the chain of 32 square roots and reciprocals of a launch (3.7 of its 10
 // us at n = 600), then the latency of its loads.  All launches, n = 15 / 143 /
-// 301 / 600 / 1024: 13 / 47 / 92 / 194 / 414 us; with a row per lane in global
+// 301 / 600 / 1024: 13 / 47 / 92 / 178 / 313 us; with a row per lane in global
 // memory too (64 lines to a load) and the update on the vector unit, its operands
 // broadcast from LDS, 20 / 114 / 251 / 413 / 775; on one workgroup 1809 us at n =
 // 600, 6768 at n = 1024.
@@ -553,45 +553,46 @@ __device__ void chol_update(const FactorArgs& a, int s, int r0, int c0, CholShar
     }
 }
 
-// v_j of block column s - 1 (loading_of's sum): the workgroup loads and
-// multiplies kLoadRows rows at a time, the next ones on their way, and a lane per
-// column adds them up.
-__device__ void chol_loading(const FactorArgs& a, int s, CholShared& sh) {
-  const int n = a.n, c = threadIdx.x % kBlk, k0 = kBlk * (s - 1);
+// v = L^T w (loading_of's sums) in pieces: piece k of block column b, its rows
+// kLoadRows k .. from the diagonal block on, is launch b + 1 + k's, which adds it
+// to what v holds of the pieces before.  Every piece up to the last block column's
+// (factor_finish) has a launch, as a block column has one for each 32 of its
+// rows.  The workgroup loads and multiplies, a lane per column adds up.  (One
+// workgroup for a whole block column took longer than the panels: 11 us of a
+// launch at n = 600, 17 at n = 1024.)
+__host__ __device__ inline int chol_load_wgs(int n, int s) {
+  // pieces k < s of block columns s - 1 - k with a row below n
+  const int k = (n - kBlk * (s - 1) + kLoadRows - kBlk - 1) / (kLoadRows - kBlk);
+  return s < k ? s : k;
+}
+__device__ void chol_loading(const FactorArgs& a, int s, int k, CholShared& sh) {
+  const int n = a.n, c = threadIdx.x % kBlk, k0 = kBlk * (s - 1 - k), i0 = k0 + kLoadRows * k;
   const double* __restrict__ col = a.L + k0 + c;
   constexpr int kPer = kLoadRows * kBlk / 256;
-  double l[kPer], w[kPer], sum = 0.0;
-  auto load = [&](int i0) {
+  double l[kPer], w[kPer];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int i = i0 + 8 * u + threadIdx.x / kBlk;
-      const bool on = i < n && i >= k0 + c;
-      l[u] = on ? col[(size_t)i * n] : 0.0;
-      w[u] = on ? a.w[i] : 0.0;
-    }
-  };
-  load(k0);
-  for (int i0 = k0; i0 < n; i0 += kLoadRows) {
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) sh.prod[8 * u + threadIdx.x / kBlk][c] = l[u] * w[u];
-    __syncthreads();
-    load(i0 + kLoadRows);
-    if (threadIdx.x < kBlk) {
-      // rows above the diagonal are zeros here, and adding one changes nothing
-      const int m = min(kLoadRows, n - i0);
-      int i = 0;
-      for (; i + 16 <= m; i += 16) {
-        double p[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) p[u] = sh.prod[i + u][c];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) sum += p[u];
-      }
-      for (; i < m; ++i) sum += sh.prod[i][c];
-    }
-    __syncthreads();
+  for (int u = 0; u < kPer; ++u) {
+    const int i = i0 + 8 * u + threadIdx.x / kBlk;
+    const bool on = i < n && i >= k0 + c;
+    l[u] = on ? col[(size_t)i * n] : 0.0;
+    w[u] = on ? a.w[i] : 0.0;
   }
-  if (threadIdx.x < kBlk) a.v64[k0 + c] = sum;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) sh.prod[8 * u + threadIdx.x / kBlk][c] = l[u] * w[u];
+  __syncthreads();
+  if (threadIdx.x < kBlk) {
+    // the entries above the diagonal and past row n are zeros here, and adding
+    // one changes nothing
+    double sum = k == 0 ? 0.0 : a.v64[k0 + c];
+    for (int i = 0; i < kLoadRows; i += 32) {
+      double p[32];
+#pragma unroll
+      for (int u = 0; u < 32; ++u) p[u] = sh.prod[i + u][c];
+#pragma unroll
+      for (int u = 0; u < 32; ++u) sum += p[u];
+    }
+    a.v64[k0 + c] = sum;
+  }
 }
 
 // The place above the diagonal where block s waited (s >= 2).
@@ -626,7 +627,7 @@ __host__ __device__ inline int chol_panel_wgs(int n, int s) {
 __host__ __device__ inline int chol_step_wgs(int n, int s) {
   if (kBlk * s >= n) return 0;
   const int t = s == 0 ? (n + 63) / 64 : (n - kBlk * (s + 1) + 63) / 64;
-  return chol_panel_wgs(n, s) + (t > 0 ? (s == 0 ? t * t : t * (t + 1) / 2) : 0) + (s > 0 ? 1 : 0);
+  return chol_panel_wgs(n, s) + (t > 0 ? (s == 0 ? t * t : t * (t + 1) / 2) : 0) + (s > 0 ? chol_load_wgs(n, s) : 0);
 }
 
 __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
@@ -647,12 +648,14 @@ __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
     chol_upper(a, 64 * (t / nt), 64 * (t % nt));
     return;
   }
-  if ((int)blockIdx.x == np) {
-    chol_loading(a, s, sh);
-    if (s > 2) chol_clear(a, s - 1);
+  const int nl = chol_load_wgs(n, s);
+  if ((int)blockIdx.x < np + nl) {
+    const int k = blockIdx.x - np;
+    chol_loading(a, s, k, sh);
+    if (k == 0 && s > 2) chol_clear(a, s - 1);
     return;
   }
-  const int t = blockIdx.x - np - 1;
+  const int t = blockIdx.x - np - nl;
   int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
   while (bi * (bi + 1) / 2 > t) --bi;
   while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
