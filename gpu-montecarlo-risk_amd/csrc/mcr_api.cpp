@@ -1363,7 +1363,7 @@ uint64_t batch_signature(const mcr_query* qs, const BatchPlan& bp, int grid, int
 int enqueue_batch(const BatchPlan& bp, char* dev, char* hout, int grid, int streams) {
   const FactorArgs* fa = (const FactorArgs*)(dev + bp.offFa);
   const PrepArgs* pa = (const PrepArgs*)(dev + bp.offPa);
-  HIP_TRY(launch_factor_batch(fa, bp.nq, bp.max_n, g_ctx.stream));
+  HIP_TRY(launch_factor_batch(fa, bp.nq, bp.max_n, bp.max_n, g_ctx.stream));
   HIP_TRY(launch_prep_batch(pa, bp.nq, bp.max_n, g_ctx.stream));
   MCR_TRY(launch_runs(bp.runs, (const PathArgs*)(dev + bp.offQa),
                       (const WorkItem*)(dev + bp.offItems), (unsigned*)(dev + bp.offNext), grid,

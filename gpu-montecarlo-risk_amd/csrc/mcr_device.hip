@@ -565,8 +565,8 @@ __host__ __device__ inline int chol_load_wgs(int n, int s) {
   const int k = (n - kBlk * (s - 1) + kLoadRows - kBlk - 1) / (kLoadRows - kBlk);
   return s < k ? s : k;
 }
-__device__ void chol_loading(const FactorArgs& a, int s, int k, CholShared& sh) {
-  const int n = a.n, c = threadIdx.x % kBlk, k0 = kBlk * (s - 1 - k), i0 = k0 + kLoadRows * k;
+__device__ void chol_loading(const FactorArgs& a, int b, int k, CholShared& sh) {
+  const int n = a.n, c = threadIdx.x % kBlk, k0 = kBlk * b, i0 = k0 + kLoadRows * k;
   const double* __restrict__ col = a.L + k0 + c;
   constexpr int kPer = kLoadRows * kBlk / 256;
   double l[kPer], w[kPer];
@@ -632,7 +632,20 @@ __host__ __device__ inline int chol_step_wgs(int n, int s) {
 
 __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
   const int n = a.n, np = chol_panel_wgs(n, s);
-  if ((int)blockIdx.x >= chol_step_wgs(n, s) || a.reuse) return;
+  if ((int)blockIdx.x >= chol_step_wgs(n, s)) return;
+  if (a.reuse) {
+    // L is there from an earlier launch: the first panels' workgroups take a
+    // block column's loading each, the last one left to factor_finish (where all
+    // of them took 90 us of a serving round's setup at n = 600)
+    const int b = blockIdx.x;
+    if (s == 0 && kBlk * (b + 1) < n) {
+      for (int k = 0; kBlk * b + kLoadRows * k < n; ++k) {
+        if (k > 0) __syncthreads();
+        chol_loading(a, b, k, sh);
+      }
+    }
+    return;
+  }
   if (s > 0) {
     // one read for the workgroup: the first one may be writing it
     if (threadIdx.x == 0) sh.failed = a.info->fail_col;
@@ -651,7 +664,7 @@ __device__ void chol_step(const FactorArgs& a, int s, CholShared& sh) {
   const int nl = chol_load_wgs(n, s);
   if ((int)blockIdx.x < np + nl) {
     const int k = blockIdx.x - np;
-    chol_loading(a, s, k, sh);
+    chol_loading(a, s - 1 - k, k, sh);
     if (k == 0 && s > 2) chol_clear(a, s - 1);
     return;
   }
@@ -687,7 +700,7 @@ __device__ void factor_finish(const FactorArgs& a, FactorShared<MAXN>& sh) {
 
   int attempts = 1, clamped = 0, last_fail = 0;
   double delta = 0.0;
-  int j0 = 0;
+  int j0 = kBlk * ((a.n - 1) / kBlk);  // the launches left this block column's loading
   if (a.reuse) {
     // L holds this covariance's factor from an earlier launch.
     const DevInfo fi = *a.finfo;
@@ -707,10 +720,9 @@ __device__ void factor_finish(const FactorArgs& a, FactorShared<MAXN>& sh) {
   } else if (a.info->fail_col != 0 || !isfinite(a.A[0])) {
     __syncthreads();  // the record is read before anyone writes it
     if (!cholesky_body(a, sh, &attempts, &clamped, &last_fail, &delta)) return;
-  } else {
-    const int last = (a.n - 1) / kBlk;  // the launches left this block column's loading
-    j0 = kBlk * last;
-    if (last > 1) chol_clear(a, last);
+    j0 = 0;
+  } else if (j0 > kBlk) {
+    chol_clear(a, j0 / kBlk);
   }
   if (a.finfo && !a.reuse && tid == 0) {
     a.finfo->attempts = attempts;
@@ -748,10 +760,12 @@ hipError_t launch_factor(const FactorArgs& a, hipStream_t stream) {
 
 // max_n: the batch's largest query (a panel of 78 KiB up to kMaxN, 99 KiB
 // up to kBatchMaxN)
-hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStream_t stream) {
-  if (max_n < 1 || max_n > kBatchMaxN) return hipErrorInvalidValue;
-  for (int s = 0; kBlk * s < max_n; ++s)
-    hipLaunchKernelGGL(k_chol_step_batch, dim3(chol_step_wgs(max_n, s), nq), dim3(256), 0, stream, fas, s);
+hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, int fresh_n,
+                               hipStream_t stream) {
+  if (max_n < 1 || max_n > kBatchMaxN || fresh_n > max_n) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_chol_step_batch, dim3(chol_step_wgs(max_n, 0), nq), dim3(256), 0, stream, fas, 0);
+  for (int s = 1; kBlk * s < fresh_n; ++s)
+    hipLaunchKernelGGL(k_chol_step_batch, dim3(chol_step_wgs(fresh_n, s), nq), dim3(256), 0, stream, fas, s);
   if (max_n <= kMaxN)
     hipLaunchKernelGGL(k_factor_batch<kMaxN>, dim3(nq), dim3(1024), 0, stream, fas);
   else

@@ -148,7 +148,10 @@ struct CollectArgs {
 hipError_t launch_factor(const FactorArgs& a, hipStream_t stream);
 hipError_t launch_prep(const PrepArgs& a, hipStream_t stream);
 hipError_t launch_collect(const CollectArgs& a, hipStream_t stream);
-hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, hipStream_t stream);
+// max_n: the largest n of the queries; fresh_n: of those that do not reuse a
+// factor (0: none)
+hipError_t launch_factor_batch(const FactorArgs* fas, int nq, int max_n, int fresh_n,
+                               hipStream_t stream);
 hipError_t launch_prep_batch(const PrepArgs* pas, int nq, int max_n, hipStream_t stream);
 
 // Batched persistent execution: work item = a run of 64-path groups of one query.

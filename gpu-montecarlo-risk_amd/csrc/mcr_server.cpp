@@ -720,7 +720,7 @@ int mcr_server::enqueue_round(RoundRec& rr, const std::vector<Job*>& fresh,
   FactorArgs* fa = (FactorArgs*)(h + o_fa);
   PrepArgs* pa = (PrepArgs*)(h + o_pa);
   PathArgs* qa = (PathArgs*)(h + o_qa);
-  int max_n = 1;
+  int max_n = 1, fresh_n = 0;
   for (size_t i = 0; i < nf; ++i) {
     Job* j = fresh[i];
     const mcr_query* q = &j->q;
@@ -779,6 +779,7 @@ int mcr_server::enqueue_round(RoundRec& rr, const std::vector<Job*>& fresh,
     a.hist = d_hist;
     qa[i] = a;
     max_n = std::max(max_n, q->n);
+    if (!j->hit) fresh_n = std::max(fresh_n, q->n);
   }
   char* dr = d_round[p];
   for (size_t i = 0; i < nf; ++i) {
@@ -791,7 +792,7 @@ int mcr_server::enqueue_round(RoundRec& rr, const std::vector<Job*>& fresh,
   if (nf) {
     HIP_TRY(hipMemcpyAsync(dr + off_fa, fa, nf * sizeof(FactorArgs), hipMemcpyHostToDevice, s_setup));
     HIP_TRY(hipMemcpyAsync(dr + off_pa, pa, nf * sizeof(PrepArgs), hipMemcpyHostToDevice, s_setup));
-    HIP_TRY(launch_factor_batch((const FactorArgs*)(dr + off_fa), (int)nf, max_n, s_setup));
+    HIP_TRY(launch_factor_batch((const FactorArgs*)(dr + off_fa), (int)nf, max_n, fresh_n, s_setup));
     HIP_TRY(launch_prep_batch((const PrepArgs*)(dr + off_pa), (int)nf, max_n, s_setup));
   }
   if (!items.empty())

@@ -98,6 +98,22 @@ def test_cache_does_not_change_results(mcr):
         same(a, b)
 
 
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 65, 128, 160, 161, 300, 767])
+def test_cached_factor_with_other_weights(mcr, n):
+    """A query served on a kept factor, alone in its round or beside one that
+    brings a covariance: its loading, a workgroup per 32 columns in pieces of 128
+    rows, is the one of the query run alone."""
+    first, other = stream(60 + n, 2, sizes=(n,), reuse=0.0)
+    again = dict(first, weights=np.random.default_rng(n).dirichlet(np.ones(n)))
+    with mcr.Server() as srv:
+        same(srv.wait(srv.submit(first))[0], alone(mcr, first))
+        same(srv.wait(srv.submit(again))[0], alone(mcr, again))
+        tickets = [srv.submit(p) for p in (again, other)]
+        for p, t in zip((again, other), tickets):
+            same(srv.wait(t)[0], alone(mcr, p))
+        assert srv.stats().cache_hits >= 2
+
+
 def test_admission_budget_holds(mcr):
     ps = stream(3, 20, sizes=(100, 333, 600), reuse=0.0, paths=(5_000, 40_000))
     need = max(mcr.server_footprint(p) for p in ps)
