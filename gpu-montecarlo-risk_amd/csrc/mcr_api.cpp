@@ -931,7 +931,7 @@ void fill_statistics(int64_t M, const DevInfo& info, const DevAccum& acc, mcr_re
 
 // ---------------------------------------------------------------------------
 // Batches: batched factor (one workgroup per query), batched prepare, then one
-// persistent launch of k_batch_paths over (query, 64-path group run) work
+// persistent launch per kernel class (k_batch_small, _stage, _spec) over (query, 64-path group run) work
 // items, optionally captured once in a hipGraph and replayed.
 // ---------------------------------------------------------------------------
 // Tuned workgroup shape per row-tile range of the LDS MFMA batch kernel

@@ -998,8 +998,26 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
     return hipGetLastError();
   }
   if (kernel == 4) {
+    if (a.n > kMfmaLdsMaxN) return hipErrorInvalidValue;
+    if (a.T > 4 && a.T <= kStageMaxT) {
+      const StageShape s = stage_shape(a.n, a.T, a.S);
+      static bool attr = false;
+      if (!attr) {
+        // the largest dynamic request of each: whole chunks and the histogram
+        for (int T : {8, kStageMaxT}) {
+          const int waves = stage_waves(T), max_dyn = stage_cap(waves) * 4096 + (32 * T + 4) * 4;
+          const hipError_t e = hipFuncSetAttribute((const void*)stage_shape(32 * T - 1, T, 2 * T).kernel,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, max_dyn);
+          if (e != hipSuccess) return e;
+        }
+        attr = true;
+      }
+      const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * s.per_cu);
+      hipLaunchKernelGGL(s.kernel, dim3((unsigned)blocks), dim3(64 * s.waves), s.lds, stream, a);
+      return hipGetLastError();
+    }
     PathKernel k = mfma_big_kernel(a.T);
-    if (!k || a.n > kMfmaLdsMaxN) return hipErrorInvalidValue;
+    if (!k) return hipErrorInvalidValue;
     const int block = 64 * big_waves(a.T);
     const uint64_t per_cu = (uint64_t)resident_blocks((const void*)k, block);
     const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * per_cu);

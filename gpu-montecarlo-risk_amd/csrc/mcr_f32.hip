@@ -111,34 +111,8 @@ __global__ __launch_bounds__(64 * NW, 4) void k_f32_lds(PathArgs a) {
   }
   if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
 
-  // The deal (wave w runs on SIMD w % 4): tiles in descending order to the SIMD
-  // with the least work so far that has a slot free, there to its waves in
-  // turn (tile T-1, with the loss row: wave 0, slot 1).
-  int tile[kSlots] = {-1, -1};  // slot 1: the wave's first (larger) tile
-  {
-    int load[4] = {0, 0, 0, 0}, cnt[4] = {0, 0, 0, 0};
-    for (int tt = T - 1; tt >= 0; --tt) {
-      int s = -1, best = 1 << 30;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (cnt[k] < kSlots * NW / 4 && load[k] < best) {
-          s = k;
-          best = load[k];
-        }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (k == s) {
-          // the waves take their second tiles in reverse order
-          const int q = cnt[k], w = q < NW / 4 ? q : kSlots * NW / 4 - 1 - q;
-          if (k + 4 * w == wave) tile[q < NW / 4 ? 1 : 0] = tt;
-          load[k] += tt + 1;
-          cnt[k] = q + 1;
-        }
-      }
-    }
-  }
-  tile[0] = __builtin_amdgcn_readfirstlane(tile[0]);
-  tile[1] = __builtin_amdgcn_readfirstlane(tile[1]);
+  int tile[kSlots];  // slot 1: the wave's first (larger) tile, T - 1 wave 0's
+  deal_tiles<NW, kSlots>(T, wave, tile);
   // octets each slot runs: none, or its columns (0 <= end0 <= end1)
   const int end0 = tile[0] < 0 ? 0 : min(4 * tile[0] + 4, S);
   const int end1 = tile[1] < 0 ? 0 : min(4 * tile[1] + 4, S);

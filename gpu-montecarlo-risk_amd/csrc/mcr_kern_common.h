@@ -318,6 +318,38 @@ __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t w[4]) {
   return __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
 }
 
+// The row tiles of wave `wave` of NW (wave w runs on SIMD w % 4), at most SLOTS:
+// tiles in descending order to the SIMD with the least work so far (tile t is
+// t + 1 units) that has a slot free, there to its waves in turn.  tile[SLOTS - 1]
+// is the wave's first (larger) one, -1 a free slot; tile T - 1 is wave 0's first.
+template <int NW, int SLOTS>
+__device__ __forceinline__ void deal_tiles(int T, int wave, int (&tile)[SLOTS]) {
+  static_assert(SLOTS == 2, "a wave's two tiles");
+  tile[0] = tile[1] = -1;
+  int load[4] = {0, 0, 0, 0}, cnt[4] = {0, 0, 0, 0};
+  for (int tt = T - 1; tt >= 0; --tt) {
+    int s = -1, best = 1 << 30;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (cnt[k] < SLOTS * NW / 4 && load[k] < best) {
+        s = k;
+        best = load[k];
+      }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (k == s) {
+        // the waves take their second tiles in reverse order
+        const int q = cnt[k], w = q < NW / 4 ? q : SLOTS * NW / 4 - 1 - q;
+        if (k + 4 * w == wave) tile[q < NW / 4 ? 1 : 0] = tt;
+        load[k] += tt + 1;
+        cnt[k] = q + 1;
+      }
+    }
+  }
+  tile[0] = __builtin_amdgcn_readfirstlane(tile[0]);
+  tile[1] = __builtin_amdgcn_readfirstlane(tile[1]);
+}
+
 typedef void (*PathKernel)(PathArgs);
 PathKernel reg_kernel(int n);          // mcr_reg.hip
 PathKernel wave_kernel(int T);         // mcr_wave.hip
@@ -329,6 +361,19 @@ struct F32Shape {
   size_t lds;
 };
 F32Shape f32_shape(int n);
+// mcr_stage.hip
+// Steps that fit the LDS of one of the four (4 waves) or two (8) workgroups of a
+// compute unit; a longer S is taken in equal chunks, the sums staying in registers.
+__host__ __device__ constexpr int stage_cap(int waves) { return waves == 4 ? 9 : 19; }
+constexpr int kStageMaxT = 16;  // row tiles
+struct StageShape {
+  PathKernel kernel;
+  int waves, per_cu;
+  size_t lds;
+};
+StageShape stage_shape(int n, int T, int S);
+int stage_waves(int T);
+BatchKernel batch_stage_kernel(int T);
 PathKernel mfma_big_kernel(int T);     // mcr_mfma_big.hip
 
 }  // namespace mcr

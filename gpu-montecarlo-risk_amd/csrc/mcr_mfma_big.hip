@@ -16,9 +16,9 @@
 // Philox block (4 normals of one path) and writes its bf16 hi/lo parts
 // straight into a double-buffered LDS tile already in B-operand order, so the
 // next phase is generated while this one is multiplied; factor fragments
-// stream from L2.  For n >= 384 (13-24 row tiles; batches from 17 tiles) the
-// roles are split instead: 8 waves only multiply, 4 only generate
-// (k_mfma_spec below).
+// stream from L2.  From 17 row tiles (n >= 512) the roles are split instead: 8
+// waves only multiply, 4 only generate (k_mfma_spec below).  5 to 16 tiles run
+// mcr_stage.hip's kernel, the ones here being the batch autotuner's alternatives.
 #include "mcr_kern_common.h"
 
 namespace mcr {
@@ -536,25 +536,13 @@ hipError_t launch_batch_kernel(BatchKernel k, const BatchArgs& b, int grid, int 
   return hipGetLastError();
 }
 
-// Shapes of the LDS MFMA kernels for T row tiles (measured best per range).
-// Four waves with up to 3 tiles each for T <= 12 (several workgroups per CU,
-// so one's barrier waits are covered by another's work); beyond, single
-// queries run the split form: 8 multiplying waves of 2 (T <= 16) or 3 tiles
-// beside 4 generating waves (n = 450: 6.0 ms against 6.4 ms for eight waves of
-// 2 tiles; n = 600: 14.85 ms against 15.0 ms for 12 multiplying waves of 2
-// tiles and 16.8 ms for eight waves of 3 tiles that all generate).  The 3-tile
-// split form runs 4 K steps per phase: half the workgroup barriers of 2-step
-// phases, 0.5-1.7 % faster for n = 400-600 in interleaved timings (6- and
-// 8-step phases no faster; the 2-tile form gained at n = 450-500 and lost at
-// n = 400, so it keeps 2-step phases).  Batches
-// keep eight waves of 2 tiles at four waves per SIMD for 13-16 tiles (a
-// persistent workgroup there runs many short work items, and two per CU cover
-// each other's item changes; the 8 + 4 split form, one workgroup per CU, made
-// the uneven batch 3 % slower, and 12 + 4 waves of 1 tile for 9-12 tiles as
-// well 10 %), and the single-query shape beyond.  The split form
-// loses below 13 tiles (12 + 4 waves of 1 tile: +3 % at n = 300; 8 + 4 of 2:
-// +5 %; 4 + 4 of 3: +9 %).
-int big_waves(int T) { return T <= 12 ? 4 : 8 + kProducers; }
+// Past 16 row tiles the split form runs: 8 multiplying waves of 3 tiles beside 4
+// generating waves, 4 K steps per phase (n = 600, 1e7 paths: 14.85 ms against 15.0
+// for 12 multiplying waves of 2 tiles and 16.8 for eight waves of 3 tiles that all
+// generate; 4 K steps against 2 0.5-1.7 % faster for n = 400-600, 6 and 8 no
+// better).  5 to 16 tiles are mcr_stage.hip's; up to 4 only a caller's choice of
+// this kernel comes here.
+int big_waves(int T) { return T <= 4 ? 4 : 8 + kProducers; }
 
 // Batch shapes per row-tile range, the measured default first, then the
 // alternatives the batch autotuner may choose (every shape gives the same
@@ -565,9 +553,9 @@ struct BigShape {
   int waves;
 };
 static const BigShape kBigShapes[kBigRanges][kMaxBigShapes] = {
-    {{k_batch_paths<2, 4, false>, 4}, {k_batch_paths<1, 8, true>, 8}},
-    {{k_batch_paths<3, 4, false>, 4}, {k_batch_paths<2, 8, false>, 8}},
-    {{k_batch_paths<2, 8, false>, 8}, {k_batch_spec<8, 2, 2>, 8 + kProducers}},
+    {{batch_stage_kernel(8), stage_waves(8)}, {k_batch_paths<2, 4, false>, 4}},
+    {{batch_stage_kernel(12), stage_waves(12)}, {k_batch_paths<3, 4, false>, 4}},
+    {{batch_stage_kernel(16), stage_waves(16)}, {k_batch_paths<2, 8, false>, 8}},
     {{k_batch_spec<8, 3, 4>, 8 + kProducers}, {k_batch_spec<12, 2, 2>, 12 + kProducers}},
 };
 
@@ -587,10 +575,7 @@ BatchKernel batch_big_kernel(int T, int shape) {
 
 PathKernel mfma_big_kernel(int T) {
   if (T <= 4) return k_mfma_big<1, 4, true>;
-  if (T <= 8) return k_mfma_big<2, 4, false>;
-  if (T <= 12) return k_mfma_big<3, 4, false>;
-  if (T <= 16) return k_mfma_spec<8, 2, 2>;
-  return T <= 24 ? k_mfma_spec<8, 3, 4> : nullptr;
+  return T > kStageMaxT && T <= 24 ? k_mfma_spec<8, 3, 4> : nullptr;
 }
 
 }  // namespace mcr

@@ -17,7 +17,7 @@
 //           (factorisation skipped on a cache hit), k_prep_batch, H2D of the round's work
 //           items; event setup[p].  Overlaps the previous round's path kernel.
 //   paths:  wait setup[p]; k_batch_clear; one persistent launch per kernel class
-//           over the round's items (k_batch_small / k_batch_paths / k_batch_spec),
+//           over the round's items (k_batch_small / k_batch_stage / k_batch_spec),
 //           the classes forked over nfork streams and joined back; events
 //           start[p], end[p].
 //   out:    on the path stream after end[p]: D2H of the records of queries

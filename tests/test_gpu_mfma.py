@@ -68,6 +68,31 @@ def test_mfma_lds_vs_fp64_same_stream(mcr, orc, n, M):
     assert abs(r.var[0] - v64) <= 1e-4 * abs(v64), (r.var[0], v64)
 
 
+@pytest.mark.parametrize("n", [128, 143, 144, 145, 159, 160, 255, 256, 303, 304, 305, 319, 320, 383,
+                               384, 479, 480, 511])
+def test_mfma_staged_edges(mcr, orc, n):
+    """The kernel that stages all normals of 64 paths, at the edges of its row
+    tiles, its chunks of the K steps and its two workgroup sizes, over a range
+    of paths that crosses a multiple of 2^32 inside a group and ends inside one:
+    the tolerances above against FP64, the S histogram, and the same values
+    for the paths behind the crossing whichever group they come in."""
+    M, seed, x, k, off = 2_100, 12, 0.02, max(1, n // 5), (1 << 32) - 100
+    mu, sigma = factor_like(n, min(20, n), 70 + n, T=max(4000, 2 * n))
+    kw = dict(precision=mcr.PREC_BF16X3, want_S=True, want_loss=True)
+    r = mcr.run(mu, sigma, x, k, M, seed, path_offset=off, alphas=(0.95,), want_hist=True, **kw)
+    assert r.kernel == "mfma_lds"
+    L, *_ = mcr.factor(sigma)
+    ref = orc.simulate_f64(L, mu, np.full(n, 1.0 / n), x, seed, off, M, k, want_S=True, want_loss=True,
+                           nthreads=8)
+    assert abs(r.count - ref["count"]) <= max(3, 1e-4 * ref["count"]), (r.count, ref["count"])
+    assert np.mean(r.S != ref["S"]) <= 2e-3
+    assert np.array_equal(np.bincount(r.S, minlength=n + 1), r.s_hist)
+    v64 = np.sort(ref["loss"])[rank_of(0.95, M) - 1]
+    assert abs(r.var[0] - v64) <= 1e-4 * abs(v64), (r.var[0], v64)
+    behind = mcr.run(mu, sigma, x, k, M - 100, seed, path_offset=1 << 32, **kw)
+    assert np.array_equal(r.S[100:], behind.S) and np.array_equal(r.loss[100:], behind.loss)
+
+
 @pytest.mark.parametrize("n,M,kernel", [(50, 300_000, 3), (50, 200_000, 4), (600, 50_000, 4),
                                         (767, 20_000, 4)])
 def test_mfma_s_histogram_matches_per_path_counts(mcr, n, M, kernel):
