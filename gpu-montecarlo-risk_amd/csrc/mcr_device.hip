@@ -359,9 +359,9 @@ __device__ __forceinline__ f64x4 chain16(const double (&va)[64][LD], int ra,
 // correction of each by its fused residual ("Computation of elementary functions
 // on the IBM RISC System/6000 processor", 1990); the reciprocal starts from the
 // root's instead of an estimate of its own.  The same bits as sqrt(d) and 1.0 /
-// sqrt(d) over 2e8 random, square and near-square d, but for the reciprocal of a
-// root whose significand is all ones (d the last double below a power of four),
-// one unit in the last place off.
+// sqrt(d) over 2e8 random, square and near-square d, except where the root's
+// significand is all ones (below): there the corrected reciprocal is a tie that
+// rounds to even, one unit in the last place low.
 struct RootRecip {
   double d, g, h, q, e;
   static constexpr int kStages = 10;
@@ -379,8 +379,15 @@ struct RootRecip {
   }
 };
 
+// d is one of the last two doubles below a power of four, whose root rounds to
+// the last double below a power of two.
+__device__ __forceinline__ bool root_all_ones(double d) {
+  return (__builtin_bit_cast(uint64_t, d) & 0x001ffffffffffffeull) == 0x000ffffffffffffeull;
+}
+
 // Columns q .. q + 15 of the panel, a row per lane (rows 0-31 the diagonal
 // block's): x the row's entries, piv the pivot of the lane's column as found.
+// Not for columns with a root_all_ones pivot.
 // One wave runs this alone, so instruction order is what hides latency: the next
 // column takes its update first, and a step of its root stands before each of
 // the other columns' updates.  All launches, n = 143 / 301 / 600: 47 / 92 / 194
@@ -481,12 +488,19 @@ __device__ void chol_panel(const FactorArgs& a, int s, int blk, CholShared& sh) 
     __syncthreads();
     if (wave == 0) {
       double y[kPanel];
+      bool any = !mid;
+      if (mid) {
 #pragma unroll
-      for (int c = 0; c < kPanel; ++c) y[c] = sh.p.x[lane][kPanel * h + c];
-      if (mid)
+        for (int c = 0; c < kPanel; ++c) y[c] = sh.p.x[lane][kPanel * h + c];
         chol_columns(y, kPanel * h, &piv);
-      else
+        // the first such pivot is right, as the columns before it are
+        any = __ballot(root_all_ones(piv)) != 0ull;
+      }
+      if (any) {
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c) y[c] = sh.p.x[lane][kPanel * h + c];
         chol_columns_any(y, kPanel * h, &piv);
+      }
 #pragma unroll
       for (int c = 0; c < kPanel; ++c) sh.p.x[lane][kPanel * h + c] = y[c];
     }

@@ -123,6 +123,27 @@ def test_factor_scales_with_the_covariance(mcr, n, exp):
     assert np.array_equal(L, np.ldexp(L0, exp // 2))
 
 
+@pytest.mark.parametrize("below", [1.0, 2.0, 4.0])
+@pytest.mark.parametrize("exp", [-300, -2, 0, 8, 400])
+def test_factor_root_and_reciprocal_are_correctly_rounded(mcr, below, exp):
+    """L_jj = sqrt(d_j) and, beside a power of two c, L_nj = c (1 / sqrt(d_j)), bit
+    for bit, for the last doubles below powers of two and four (a root whose
+    significand is all ones has the one reciprocal that a fused correction rounds
+    the wrong way), in both 16-column halves of two launches."""
+    d, x = [], below
+    for _ in range(40):
+        x = np.nextafter(x, 0.0)
+        d.append(np.ldexp(x, exp))
+    d = np.array(d)
+    c = np.ldexp(1.0, exp - 8)
+    A = np.diag(np.append(d, np.ldexp(1.0, exp)))
+    A[-1, :-1] = A[:-1, -1] = c
+    L, att, jit, cl = mcr.factor(A)
+    assert (att, jit, cl) == (1, 0.0, 0)
+    assert np.array_equal(np.diag(L)[:-1], np.sqrt(d))
+    assert np.array_equal(L[-1, :-1], c * (1.0 / np.sqrt(d)))
+
+
 def test_factor_clamp_fallback(mcr, orc):
     A = np.diag([1.0, 1.0, -0.5, 1.0]) * 1e-4
     L, att, jit, cl = mcr.factor(A)
