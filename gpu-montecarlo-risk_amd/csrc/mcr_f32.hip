@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_f32_lds(PathArgs a) {
   extern __shared__ float4 zs[];  // [octet - chunk start][path half][64]
   __shared__ int sS[NW][64];
   __shared__ float sLoss[64];
-  __shared__ LdsTally t;
+  __shared__ LdsTally<1> t;
   const int n = a.n, T = a.T, S = a.S;
   const int nb = (n + 3) >> 2;
   const int chunk = n <= kMaxN ? S : kChunkCols / 8;  // octets
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_f32_lds(PathArgs a) {
   if (want_hist) {
     for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
   }
-  if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
+  clear_tally(&t);
 
   int tile[kSlots];  // slot 1: the wave's first (larger) tile, T - 1 wave 0's
   deal_tiles<NW, kSlots>(T, wave, tile);
@@ -247,7 +247,7 @@ F32Shape f32_shape(int n) {
           ((n + 1) * sizeof(unsigned) + 15) / 16 * 16;
   // static LDS: counts and losses of 64 paths per wave, the tally
   auto fits = [&](int waves) {
-    const size_t stat = sizeof(int) * waves * 64 + sizeof(float) * 64 + sizeof(LdsTally);
+    const size_t stat = sizeof(int) * waves * 64 + sizeof(float) * 64 + sizeof(LdsTally<1>);
     return (int)((160 * 1024) / (s.lds + stat));
   };
   s.waves = fits(4) >= 4 ? 4 : (fits(8) >= 2 ? 8 : 16);

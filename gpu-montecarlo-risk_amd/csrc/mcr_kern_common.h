@@ -155,17 +155,34 @@ __device__ __forceinline__ void flush_tally(const PathArgs& a, const LaneTally& 
 }
 
 // The same tallies for kernels whose waves finish 64 paths at once: kept in LDS
-// (ballots and population counts, added by one lane; the few losses above a
-// window add themselves), so a path loop carries none of them in registers.
-// One record per flushing unit (a workgroup, or a wave of the batch kernels).
+// (ballots and population counts, added by one lane; the losses above a window
+// add themselves), so a path loop carries none of them in registers.  One record
+// per workgroup.  LDS takes adds to one address in turn, so kernels with the LDS
+// to spare spread the lanes' losses over SLOTS sums: at a level of 5 % 60 of the
+// 64 lanes add one.
+template <int SLOTS>
 struct LdsTally {
-  unsigned long long v[4 + 2 * kMaxAlpha];  // count, near, hist below / above,
-                                            // above[], sum_above[]
+  unsigned long long v[4 + kMaxAlpha];  // count, near, hist below / above, above[]
+  unsigned long long sum_above[kMaxAlpha][SLOTS];
 };
-constexpr int kTallyWords = 4 + 2 * kMaxAlpha;
+
+// SLOTS of the kernels for n <= 127, whose LDS is free (1e7-2e7 paths, level 5 %, 1
+// -> 16 slots: n = 8 665 -> 439 us, n = 20 805 -> 582, n = 50 715 -> 600; at 99 %
+// the same; 32 no better).  The ones past n = 127 fill it, and have a tenth of the
+// losses for their work: one.
+constexpr int kTallySlots = 16;
+
+// By a thread per word.
+template <int SLOTS>
+__device__ __forceinline__ void clear_tally(LdsTally<SLOTS>* t) {
+  constexpr int kWords = sizeof(LdsTally<SLOTS>) / 8;
+  static_assert(kWords <= 256, "a word per thread");
+  if (threadIdx.x < kWords) reinterpret_cast<unsigned long long*>(t)[threadIdx.x] = 0ull;
+}
 
 // All 64 lanes of the wave, valid marking the paths that count.
-__device__ __forceinline__ void tally_wave(const PathArgs& a, LdsTally* t, uint64_t q, bool valid,
+template <int SLOTS>
+__device__ __forceinline__ void tally_wave(const PathArgs& a, LdsTally<SLOTS>* t, uint64_t q, bool valid,
                                            int S, float loss, bool near, unsigned* sh_hist) {
   const DevInfo* ip = a.info;
   asm volatile("" : "+s"(ip));
@@ -187,7 +204,8 @@ __device__ __forceinline__ void tally_wave(const PathArgs& a, LdsTally* t, uint6
       if (al < a.n_alpha) {
         const bool above = valid && loss > w->hi[al];
         add(4 + al, above);
-        if (above) atomicAdd(&t->v[4 + kMaxAlpha + al], (unsigned long long)fixed32(loss));
+        if (above)
+          atomicAdd(&t->sum_above[al][threadIdx.x % SLOTS], (unsigned long long)fixed32(loss));
         append_loss(a, al, valid && loss >= w->lo[al] && loss <= w->hi[al], loss);
       }
     }
@@ -201,16 +219,26 @@ __device__ __forceinline__ void tally_wave(const PathArgs& a, LdsTally* t, uint6
   }
 }
 
-// Lane i of the first 12 adds word i to the query's accumulators and clears it.
-__device__ __forceinline__ void flush_tally_lds(const PathArgs& a, LdsTally* t, int i) {
-  if (i >= kTallyWords) return;
+// Lane i of the first 12 adds tally i to the query's accumulators and clears it.
+template <int SLOTS>
+__device__ __forceinline__ void flush_tally_lds(const PathArgs& a, LdsTally<SLOTS>* t, int i) {
+  if (i >= 4 + 2 * kMaxAlpha) return;
   unsigned long long* const acc = &a.acc->count;
   // DevAccum: count, near, above[], sum_above[], gathered[], hist below, hist above
   unsigned long long* dst = i < 2 ? acc + i
                             : i < 4 ? &a.acc->hist_below + (i - 2)
                                     : acc + (i - 2);
-  const unsigned long long v = t->v[i];
-  t->v[i] = 0ull;
+  unsigned long long v = 0;
+  if (i < 4 + kMaxAlpha) {
+    v = t->v[i];
+    t->v[i] = 0ull;
+  } else {
+    unsigned long long* sum = t->sum_above[i - 4 - kMaxAlpha];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) v += sum[s];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) sum[s] = 0ull;
+  }
   if (v) atomicAdd(dst, v);
 }
 

@@ -25,7 +25,7 @@ namespace mcr {
 // normals need no lane exchange and the half-wave pair shares one path.
 template <int NB, int T>
 __device__ __forceinline__ void mfma_wave_groups(const PathArgs& a, uint64_t g0, uint64_t g1,
-                                                 uint64_t gstep, LdsTally* t, unsigned* sh_hist) {
+                                                 uint64_t gstep, LdsTally<kTallySlots>* t, unsigned* sh_hist) {
   constexpr int S = (NB + 3) / 4;  // 16-wide K steps
   const int lane = threadIdx.x & 63;
   const int h = lane >> 5;
@@ -131,13 +131,13 @@ constexpr int mfma_min_waves(int T) { return T <= 2 ? 4 : 2; }
 template <int NB, int T>
 __global__ __launch_bounds__(256, mfma_min_waves(T)) void k_mfma(PathArgs a) {
   __shared__ unsigned sh_hist[32 * kMfmaMaxT];
-  __shared__ LdsTally t;
+  __shared__ LdsTally<kTallySlots> t;
   const int n = a.n;
   const bool want_hist = a.s_hist != nullptr;
   if (want_hist) {
     for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
   }
-  if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
+  clear_tally(&t);
   __syncthreads();
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x >> 6);
   mfma_wave_groups<NB, T>(a, (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6),
@@ -162,9 +162,9 @@ __global__ __launch_bounds__(256, mfma_min_waves(T)) void k_mfma(PathArgs a) {
 // the same paths 99 us on their own).
 template <int NB, int T>
 __global__ __launch_bounds__(256, mfma_min_waves(T)) void k_batch_small(BatchArgs b) {
-  __shared__ LdsTally t;
+  __shared__ LdsTally<kTallySlots> t;
   __shared__ unsigned s_next;
-  if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
+  clear_tally(&t);
   __syncthreads();
   for (unsigned it = blockIdx.x; it < b.nitems;) {
     unsigned next = 0;

@@ -82,7 +82,7 @@ template <int NW>
 struct StageShared {
   int sS[NW][64];
   float sLoss[64];
-  LdsTally t;
+  LdsTally<1> t;
 };
 
 // Groups g0, g0 + gstep, ... < g1 of 64 paths of query a; zs: [step][path half]
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_mfma_stage(PathArgs a) {
   if (want_hist) {
     for (int i = threadIdx.x; i <= a.n; i += blockDim.x) sh_hist[i] = 0u;
   }
-  if (threadIdx.x < kTallyWords) sh.t.v[threadIdx.x] = 0ull;
+  clear_tally(&sh.t);
   __syncthreads();
   stage_groups<NW>(a, blockIdx.x, (a.npaths + 63) / 64, gridDim.x, stage_z, sh,
                    want_hist ? sh_hist : nullptr);
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_batch_stage(BatchArgs b) {
   __shared__ uint4 zs[stage_cap(NW) * 256];
   __shared__ StageShared<NW> sh;
   __shared__ unsigned s_item;
-  if (threadIdx.x < kTallyWords) sh.t.v[threadIdx.x] = 0ull;
+  clear_tally(&sh.t);
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(b.next, 1u);
     __syncthreads();

@@ -111,7 +111,7 @@ __device__ __forceinline__ void stage_query(const PathArgs& a, float4* lds) {
 // accumulated into the tally t (no workgroup barriers).
 template <int T>
 __device__ __forceinline__ void wave_groups(const PathArgs& a, const float4* lds, uint64_t g0,
-                                            uint64_t g1, uint64_t gstep, LdsTally* t, unsigned* sh_hist) {
+                                            uint64_t g1, uint64_t gstep, LdsTally<kTallySlots>* t, unsigned* sh_hist) {
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const Key2 key = key_of(a.seed);
   const bool want_near = a.thr_lo < a.thr_hi;
@@ -165,13 +165,13 @@ template <int T>
 __global__ __launch_bounds__(256, wave_min_waves(T)) void k_wave(PathArgs a) {
   extern __shared__ float4 lds[];
   __shared__ unsigned sh_hist[32 * kMfmaMaxT];
-  __shared__ LdsTally t;
+  __shared__ LdsTally<kTallySlots> t;
   const int n = a.n;
   const bool want_hist = a.s_hist != nullptr;
   if (want_hist) {
     for (int i = threadIdx.x; i <= n; i += blockDim.x) sh_hist[i] = 0u;
   }
-  if (threadIdx.x < kTallyWords) t.v[threadIdx.x] = 0ull;
+  clear_tally(&t);
   stage_query<T>(a, lds);
   __syncthreads();
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x >> 6);

@@ -130,3 +130,23 @@ def test_loss_moments_reported(mcr):
     r = mcr.run(mu, sigma, 0.02, 3, 1000, 5, alphas=(0.99,))
     assert r.loss_mean == pytest.approx(-(w @ mu), rel=1e-12)
     assert r.loss_sd == pytest.approx(np.sqrt(w @ sigma @ w), rel=1e-9)
+
+
+@pytest.mark.parametrize("n,precision", [(8, "bf16x3"), (50, "bf16x3"), (100, "bf16x3"), (143, "bf16x3"),
+                                         (301, "bf16x3"), (70, "fp32"), (143, "fp32")])
+@pytest.mark.parametrize("M", [3, 65, 20_011])
+def test_tail_sums_where_most_losses_are_above_the_window(mcr, n, precision, M):
+    """Levels low enough that nearly every, half or few of a wave's 64 losses lie
+    above their windows, on the kernels that tally a wave at once: VaR and the
+    fixed-point tail sum equal those of the same call's per-path losses, negative
+    ones in the tail among them."""
+    mu, sigma = factor_like(n, 3, 60 + n, T=max(1500, 2 * n))
+    alphas = (0.01, 0.5, 0.9, 0.999)
+    r = mcr.run(mu, sigma, 0.02, 2, M, 17, precision=mcr.PREC_BF16X3 if precision == "bf16x3" else mcr.PREC_FP32,
+                alphas=alphas, want_loss=True)
+    srt = np.sort(r.loss)
+    assert M < 100 or srt[rank_of(0.01, M) - 1] < 0
+    for i, a in enumerate(alphas):
+        R = rank_of(a, M)
+        assert r.var[i] == srt[R - 1]
+        assert r.tail_sum_fixed[i] == int(np.sum((srt[R - 1:].astype(np.float64) * 2.0**32).astype(np.int64)))
