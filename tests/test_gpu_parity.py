@@ -7,7 +7,9 @@ kernels mirror the oracle's fixed fma order); FP64 factor within 1e-10
 relative of LAPACK."""
 from __future__ import annotations
 
+import ctypes
 import json
+import math
 import os
 
 import numpy as np
@@ -142,6 +144,44 @@ def test_factor_root_and_reciprocal_are_correctly_rounded(mcr, below, exp):
     assert (att, jit, cl) == (1, 0.0, 0)
     assert np.array_equal(np.diag(L)[:-1], np.sqrt(d))
     assert np.array_equal(L[-1, :-1], c * (1.0 / np.sqrt(d)))
+
+
+def _factor_replay(A):
+    """The factor by panels of 16 columns, operation by operation: inside a panel
+    one fused multiply-add per column, to the columns behind it a chain of 16 from
+    zero, then one subtraction."""
+    fma = ctypes.CDLL("libm.so.6").fma
+    fma.restype, fma.argtypes = ctypes.c_double, [ctypes.c_double] * 3
+    n = len(A)
+    L = np.tril(A).tolist()
+    for k0 in range(0, n, 16):
+        k1 = min(k0 + 16, n)
+        for c in range(k0, k1):
+            root = math.sqrt(L[c][c])
+            rl = 1.0 / root
+            L[c][c] = root
+            for r in range(c + 1, n):
+                L[r][c] *= rl
+            for r in range(c + 1, n):
+                for c2 in range(c + 1, min(r + 1, k1)):
+                    L[r][c2] = fma(-L[r][c], L[c2][c], L[r][c2])
+        for i in range(k1, n):
+            for j in range(k1, i + 1):
+                acc = 0.0
+                for p in range(k0, k1):
+                    acc = fma(L[i][p], L[j][p], acc)
+                L[i][j] -= acc
+    return np.array(L)
+
+
+@pytest.mark.parametrize("n", [17, 33, 70, 101])
+def test_factor_bits_are_its_chains_of_fused_multiply_adds(mcr, n):
+    """Every entry of the first attempt, whose updates run on the FP64 matrix
+    instruction over several launches, bit for bit as a host replay computes it."""
+    A = random_spd(n, 500 + n, cond=50.0)
+    L, att, _, _ = mcr.factor(A)
+    assert att == 1
+    assert np.array_equal(L, _factor_replay(A))
 
 
 def test_factor_clamp_fallback(mcr, orc):
