@@ -97,6 +97,7 @@ int ensure_init(int device) {
     return MCR_E_DEVICE;
   }
   g_ctx.scratch = sp;
+  HIP_TRY(init_path_kernels());
   g_ctx.ready = true;
   return MCR_OK;
 }

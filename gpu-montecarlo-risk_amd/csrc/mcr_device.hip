@@ -969,6 +969,22 @@ int resident_blocks(const void* kernel, int block, size_t lds) {
   return per_cu;
 }
 
+// The path kernels' dynamic LDS past 64 KiB, which a device takes only as an
+// attribute of the kernel: the largest request of each that has one.  Static LDS
+// comes on top (160 KiB in all).
+hipError_t init_path_kernels() {
+  auto allow = [](PathKernel k, size_t lds) {
+    return hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  };
+  hipError_t e = allow(wave_kernel(kMfmaMaxT), wave_lds(kMfmaMaxT, 4 * kMfmaMaxT));
+  for (int n : {kMaxN, 256, 128})  // 16, 8 and 4 waves
+    if (e == hipSuccess) e = allow(f32_shape(n).kernel, f32_shape(kMaxN).lds);
+  for (int T : {8, kStageMaxT})  // whole chunks and the histogram
+    if (e == hipSuccess)
+      e = allow(stage_shape(32 * T - 1, T, 2 * T).kernel, stage_cap(stage_waves(T)) * 4096 + (32 * T + 4) * 4);
+  return e;
+}
+
 hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t stream) {
   if (a.npaths == 0) return hipSuccess;
   if (kernel == 3) {
@@ -989,17 +1005,6 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
   if (a.f32 == kF32Lds) {
     if (a.n < 1 || a.n > kChunkMaxN) return hipErrorInvalidValue;
     const F32Shape s = f32_shape(a.n);
-    static bool attr = false;
-    if (!attr) {
-      // the largest dynamic request; static LDS comes on top (160 KiB in all)
-      const int max_dyn = (int)f32_shape(kMaxN).lds;
-      for (int n : {kMaxN, 256, 128}) {
-        const hipError_t e = hipFuncSetAttribute((const void*)f32_shape(n).kernel,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, max_dyn);
-        if (e != hipSuccess) return e;
-      }
-      attr = true;
-    }
     const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * s.per_cu);
     hipLaunchKernelGGL(s.kernel, dim3((unsigned)blocks), dim3(64 * s.waves), s.lds, stream, a);
     return hipGetLastError();
@@ -1015,17 +1020,6 @@ hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t 
     if (a.n > kMfmaLdsMaxN) return hipErrorInvalidValue;
     if (a.T > 4 && a.T <= kStageMaxT) {
       const StageShape s = stage_shape(a.n, a.T, a.S);
-      static bool attr = false;
-      if (!attr) {
-        // the largest dynamic request of each: whole chunks and the histogram
-        for (int T : {8, kStageMaxT}) {
-          const int waves = stage_waves(T), max_dyn = stage_cap(waves) * 4096 + (32 * T + 4) * 4;
-          const hipError_t e = hipFuncSetAttribute((const void*)stage_shape(32 * T - 1, T, 2 * T).kernel,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, max_dyn);
-          if (e != hipSuccess) return e;
-        }
-        attr = true;
-      }
       const uint64_t blocks = min_u64((a.npaths + 63) / 64, (uint64_t)num_cus * s.per_cu);
       hipLaunchKernelGGL(s.kernel, dim3((unsigned)blocks), dim3(64 * s.waves), s.lds, stream, a);
       return hipGetLastError();

@@ -189,6 +189,7 @@ hipError_t launch_batch_clear(unsigned* next, int count, hipStream_t stream);
 hipError_t launch_batch_kernel(BatchKernel k, const BatchArgs& b, int grid, int block,
                                hipStream_t stream);
 size_t wave_lds(int T, int S);  // dynamic LDS of the fp32 wave kernel
+hipError_t init_path_kernels();  // once per device, before launch_paths
 hipError_t launch_paths(int kernel, const PathArgs& a, int num_cus, hipStream_t stream);
 hipError_t launch_normals(uint64_t seed, uint64_t path0, uint64_t npaths, int n, float* out,
                           hipStream_t stream);
