@@ -21,9 +21,7 @@
 // Every path kernel reduces the exceedance count, tail counts and fixed-point
 // tail sums per lane, then per wave, with one atomic per wave per counter; no
 // normal ever leaves the chip.
-#include <map>
 #include <mutex>
-#include <tuple>
 
 #include "mcr_kern_common.h"
 
@@ -953,19 +951,29 @@ hipError_t launch_normals(uint64_t seed, uint64_t path0, uint64_t npaths, int n,
 // ---------------------------------------------------------------------------
 static uint64_t min_u64(uint64_t x, uint64_t y) { return x < y ? x : y; }
 
+// Kept in an array, not on the heap: the allocation-free entry point asks too.  It
+// holds every shape there is (about 70: a path kernel's block and LDS follow from
+// n); past its end the runtime is asked again each time.
 int resident_blocks(const void* kernel, int block, size_t lds) {
+  struct Known {
+    const void* kernel;
+    int block;
+    size_t lds;
+    int per_cu;
+  };
   static std::mutex mu;
-  static std::map<std::tuple<const void*, int, size_t>, int> cache;
+  static Known known[128];
+  static int count = 0;
   std::lock_guard<std::mutex> lk(mu);
-  auto it = cache.find({kernel, block, lds});
-  if (it != cache.end()) return it->second;
+  for (int i = 0; i < count; ++i)
+    if (known[i].kernel == kernel && known[i].block == block && known[i].lds == lds) return known[i].per_cu;
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds) != hipSuccess ||
       per_cu < 1) {
     (void)hipGetLastError();
     per_cu = 1;
   }
-  cache[{kernel, block, lds}] = per_cu;
+  if (count < (int)(sizeof(known) / sizeof(known[0]))) known[count++] = {kernel, block, lds, per_cu};
   return per_cu;
 }
 
