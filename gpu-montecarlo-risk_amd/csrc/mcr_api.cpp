@@ -972,10 +972,13 @@ int class_grid(BatchKernel k, int block) {
   return resident_blocks(reinterpret_cast<const void*>(k), block) * cus;
 }
 
-uint64_t item_groups(int n, uint64_t groups, int grid, uint64_t cap) {
-  uint64_t g = groups / (4 * (uint64_t)grid);
-  if (n <= kSmallMaxN) g = std::max<uint64_t>(4, g / 4 * 4);
-  return std::max<uint64_t>(1, std::min(g, cap));
+uint64_t item_groups(int n, uint64_t groups, int grid, uint64_t cap, double scale) {
+  const uint64_t waves = n <= kSmallMaxN ? 4 : 1;  // that share an item's groups
+  if (cap >= waves) cap -= cap % waves;
+  const uint64_t g = groups / (4 * (uint64_t)grid);
+  const uint64_t item = std::min(std::max(g - g % waves, waves), std::max<uint64_t>(cap, 1));
+  if (scale == 1.0) return item;
+  return (uint64_t)std::ceil(scale * (double)item / (double)waves) * waves;
 }
 
 void order_by_class(std::vector<WorkItem>* items, const std::vector<BatchKernel>& qk,

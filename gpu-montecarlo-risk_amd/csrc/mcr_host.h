@@ -137,9 +137,9 @@ int class_block(int n, const int* shapes = nullptr);
 int class_grid(BatchKernel k, int block);
 // Groups per work item of an n-asset query whose class has groups to run on grid
 // workgroups: four items per workgroup, so that the launch balances, at most cap
-// groups, and where the workgroup's four waves share an item (n <= 127) a
-// multiple of four, not less than four.
-uint64_t item_groups(int n, uint64_t groups, int grid, uint64_t cap);
+// groups; where the workgroup's four waves share an item (n <= 127) a multiple of
+// four, unless cap is less.  scale: times as many, where items must be fewer.
+uint64_t item_groups(int n, uint64_t groups, int grid, uint64_t cap, double scale = 1.0);
 void order_by_class(std::vector<WorkItem>* items, const std::vector<BatchKernel>& qk,
                     const std::vector<int>& qb, const std::vector<double>& qcost, bool lpt,
                     std::vector<ClassRun>* runs);

@@ -643,14 +643,14 @@ int mcr_server::plan_round(uint64_t round, RoundRec* rr, std::vector<WorkItem>* 
   tuned_shapes(shapes);
   std::map<BatchKernel, uint64_t> class_groups;
   for (auto& gr : grant) class_groups[class_kernel(gr.first->q.n, shapes)] += gr.second;
-  auto job_item_groups = [&](const Job* j) {
+  auto job_item_groups = [&](const Job* j, double scale) {
     const int n = j->q.n;
     const BatchKernel k = class_kernel(n, shapes);
-    return item_groups(n, class_groups[k], class_grid(k, class_block(n, shapes)), kItemGroups);
+    return item_groups(n, class_groups[k], class_grid(k, class_block(n, shapes)), kItemGroups, scale);
   };
   size_t est = 0;
   for (auto& gr : grant) {
-    const uint64_t ig = job_item_groups(gr.first);
+    const uint64_t ig = job_item_groups(gr.first, 1.0);
     est += (size_t)((gr.second + ig - 1) / ig);
   }
   const double scale = est > kMaxItems ? (double)est / kMaxItems + 1.0 : 1.0;
@@ -658,7 +658,7 @@ int mcr_server::plan_round(uint64_t round, RoundRec* rr, std::vector<WorkItem>* 
   for (auto& gr : grant) {
     Job* j = gr.first;
     const double c = group_cost(j->T, j->S);
-    const uint64_t ig = std::max<uint64_t>(1, (uint64_t)std::ceil(scale * (double)job_item_groups(j)));
+    const uint64_t ig = job_item_groups(j, scale);
     const uint64_t g0 = j->next_group, g1 = g0 + gr.second;
     for (uint64_t g = g0; g < g1; g += ig) {
       WorkItem w;

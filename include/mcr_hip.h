@@ -178,7 +178,8 @@ typedef struct mcr_batch_opts {
   int mode;          /* MCR_BATCH_* */
   int use_graph;     /* capture the device work in a hipGraph (replayed while the batch
                         layout is unchanged) */
-  int chunk_paths;   /* paths per work item, multiple of 64; 0 = autotuned value */
+  int chunk_paths;   /* paths per work item, at most, multiple of 64 (from 256 on a multiple
+                        of 256 for n <= 127); 0 = autotuned value */
   int order;         /* MCR_ORDER_*; used when chunk_paths != 0 */
   int grid;          /* persistent workgroups per launch; 0 = each class kernel's
                         resident maximum (occupancy x CUs) */

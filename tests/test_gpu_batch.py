@@ -105,6 +105,17 @@ def test_small_items_over_the_workgroup(mcr, chunk, grid):
         same(r, alone(mcr, p))
 
 
+@pytest.mark.parametrize("n,chunk,groups", [(8, 64, 1), (8, 192, 3), (8, 256, 4), (8, 320, 4), (8, 448, 4),
+                                            (8, 512, 8), (200, 64, 1), (200, 320, 5)])
+def test_items_are_whole_multiples_of_the_waves_that_share_them(mcr, n, chunk, groups):
+    """Item sizes in groups of 64 paths: the given limit, rounded down to a multiple
+    of four where four waves share an item and the limit allows one."""
+    total = 200_000 if n <= 127 else 60_000
+    ps = portfolios(8, sizes=(n,), paths=[64 * total])
+    _, o = mcr.run_batch(ps, use_graph=False, chunk_paths=chunk)
+    assert o.work_items == -(-total // groups)
+
+
 def test_batch_refinement_fallback(mcr):
     ps = portfolios(5, sizes=(20, 40))
     ps[1]["alphas"] = (0.95, 0.99)
