@@ -66,6 +66,18 @@ def test_batch_equals_alone_at_class_boundaries(mcr):
             same(r, alone(mcr, p))
 
 
+def test_batch_items_across_32_bits(mcr):
+    """Path ids that cross 2^32 inside a 64-path group and at a group's edge, in
+    every batch class: the results of the queries alone."""
+    ps = portfolios(13, sizes=(20, 100, 143, 300, 450, 600), paths=[6000, 5000, 4000, 3000, 3000, 2500])
+    for i, p in enumerate(ps):
+        p["path_offset"] = 2**32 - (1472 if i % 2 else 1469)
+    res, _ = mcr.run_batch(ps, use_graph=False, chunk_paths=512)
+    for p, r in zip(ps, res):
+        same(r, mcr.run(p["mu"], p["sigma"], p["x"], p["k"], p["paths"], p["seed"], weights=p["weights"],
+                        precision=mcr.PREC_BF16X3, alphas=p["alphas"], path_offset=p["path_offset"]))
+
+
 def test_graph_replay_uses_new_inputs(mcr):
     a = portfolios(2)
     b = portfolios(3, paths=[p["paths"] for p in a])  # same shapes, new data and seeds

@@ -269,6 +269,42 @@ def test_lds_kernel_exact_where_workgroups_fit(mcr, orc, n):
     _exact_case(mcr, orc, n, 1500, max(1, n // 5), 2, path_offset=2**32 - 741)
 
 
+@pytest.mark.parametrize("n", [609, 640, 1024])
+def test_column_chunks_of_a_group_across_32_bits(mcr, orc, n):
+    """The same past 608 assets, where a group whose path ids cross 2^32 goes
+    through its column chunks twice."""
+    _exact_case(mcr, orc, n, 1500, n // 5, 5, path_offset=2**32 - 741, K=12)
+
+
+@pytest.mark.parametrize("scale,x", [(1e-38, 1e-40), (1e-40, 1e-42), (3e39, 1e38), (1e41, 1e38)])
+@pytest.mark.parametrize("n,kernel", [(50, 1), (50, 2), (95, 2), (127, 2), (128, 5), (143, 2), (305, 2),
+                                      (608, 2), (640, 5)])
+def test_fp32_kernels_exact_at_the_ends_of_the_range(mcr, orc, n, kernel, scale, x):
+    """Subnormal factors and sums, overflowing sums, infinite factor entries (their
+    NaNs included) and means: S, the losses (any NaN equal to any other), the counts
+    and the histogram are the oracle's, so the matrix instruction neither flushes
+    nor reorders."""
+    mu, sigma = factor_like(n, 3, 31 + n, T=max(1500, 2 * n))
+    mu, sigma = mu * scale, sigma * scale * scale
+    if scale > 1e40:
+        mu[::3] *= -1e5  # past fp32, most to +-infinity
+        mu[1::3] = 1.0
+    model, m = device_model(mcr, orc, mu, sigma, x)
+    low = np.abs(m["L32"][np.tril_indices(n)])
+    assert np.all(low < 2.0**-126) if scale < 1 else np.any(np.isinf(low)) == (scale > 1e40)
+    k = max(1, n // 5)
+    r = mcr.run(mu, sigma, x, k, 1500, 2024, kernel=kernel, want_S=True, want_loss=True, near=True,
+                want_hist=True)
+    ref = orc.simulate_f32(model, 2024, 0, 1500, k, want_S=True, want_loss=True, want_hist=True,
+                           nthreads=8)
+    assert np.array_equal(r.S, ref["S"])
+    assert np.array_equal(np.isnan(r.loss), np.isnan(ref["loss"]))
+    ok = ~np.isnan(r.loss)
+    assert np.array_equal(r.loss[ok].view(np.uint32), ref["loss"][ok].view(np.uint32))
+    assert (r.count, r.near_threshold) == (ref["count"], ref["near"])
+    assert np.array_equal(r.s_hist, ref["hist"])
+
+
 @pytest.mark.parametrize("n", [1, 5, 9, 50, 129, 257, 600, 608, 609, 700, 1000, 1024])
 def test_chunk_kernel_exact(mcr, orc, n):
     """The column-chunk kernel (any n <= 1024; fp32 past 608): per-path
