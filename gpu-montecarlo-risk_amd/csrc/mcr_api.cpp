@@ -47,7 +47,7 @@ constexpr uint64_t kPerPathChunk = 1ull << 24;  // per-path outputs staged per l
 // Device scratch of the allocation-free entry point (mcr_run_noalloc): every
 // device buffer of one query (covariance, factor, layouts, accumulators, VaR
 // gather buffers, per-path output chunks) is carved from this array instead of
-// the arena.  16 MiB holds the largest query (15.3 MiB: n = 608, four VaR levels,
+// the arena.  16 MiB holds the largest query (13.2 MiB: n = 608, four VaR levels,
 // per-path outputs staged 2^18 paths at a time); every device the library
 // runs on holds it until the process ends.  Host code reaches it only through
 // g_ctx.scratch, its device address from hipGetSymbolAddress.
@@ -242,7 +242,7 @@ int choose_kernel(const mcr_query* q, Plan* p) {
     } else if (n <= kMfmaLdsMaxN) {
       k = n <= 32 * kMfmaMaxT - 1 ? MCR_KERNEL_MFMA : MCR_KERNEL_MFMA_LDS;
     } else {
-      // past the LDS MFMA kernel's 24 row tiles the column-chunk fp32 kernel
+      // past the LDS MFMA kernel's 24 row tiles the fp32 LDS kernel in column chunks
       // runs every precision (fp32 error is no larger than the bf16x3 products')
       k = MCR_KERNEL_VALU_CHUNK;
     }
@@ -931,9 +931,10 @@ void fill_statistics(int64_t M, const DevInfo& info, const DevAccum& acc, mcr_re
 }
 
 // ---------------------------------------------------------------------------
-// Batches: batched factor (one workgroup per query), batched prepare, then one
-// persistent launch per kernel class (k_batch_small, _stage, _spec) over (query, 64-path group run) work
-// items, optionally captured once in a hipGraph and replayed.
+// Batches: batched factor (a launch per 32 columns for all queries, then one
+// workgroup per query), batched prepare, then one persistent launch per kernel
+// class (k_batch_small, _stage, _spec) over (query, 64-path group run) work items,
+// optionally captured once in a hipGraph and replayed.
 // ---------------------------------------------------------------------------
 // Tuned workgroup shape per row-tile range of the LDS MFMA batch kernel
 // (index into the shapes of batch_big_kernel; 0 = the measured default).  The

@@ -5,9 +5,12 @@
 //   Z ~ N(0, I_N), R = mu + L Z (lower-triangular, :51-57), S = #{R_i < -x} (:60-65),
 //   extreme iff S >= k (:69-71), and stores S (:67).
 // Here:
-//   k_factor     FP64 blocked Cholesky on one workgroup with the jitter policy, then
-//                the portfolio loading v = L^T w, w^T mu and ||v|| (one launch).
+//   k_chol_step  FP64 Cholesky and the portfolio loading v = L^T w, one launch per
+//                32 columns, many workgroups.
+//   k_factor     one workgroup behind them: w^T mu and ||v||, the query's record, and
+//                the jitter policy's retries where the first attempt failed.
 //   k_prep       fp32 / bf16 layouts of the factor for the path kernels.
+//   k_collect    the query's results to pinned host memory.
 //   k_valu_reg   fused path kernel, one path per lane, n <= 64 rows in registers,
 //                factor read through the scalar cache: r_i = mu_i then fmaf(L_ij, z_j)
 //                for j = 0..i, exactly the order the C mirror uses.
@@ -18,9 +21,13 @@
 //   k_mfma       32 paths per wave on v_mfma_f32_32x32x16_bf16: A = factor rows
 //                (bf16 hi/lo), B = normals (bf16 hi/lo), three products per step
 //                (hi*hi + hi*lo + lo*hi), fp32 accumulation, n <= 127.
+//   k_mfma_stage the same products, n = 128-511: 64 paths per workgroup, all their
+//                normals staged in LDS before they are multiplied.
+//   k_mfma_spec  the same, n = 512-767: waves that multiply beside waves that generate.
 // Every path kernel reduces the exceedance count, tail counts and fixed-point
-// tail sums per lane, then per wave, with one atomic per wave per counter; no
-// normal ever leaves the chip.
+// tail sums in registers (k_valu_reg, k_mfma_spec) or LDS and adds them to the
+// query's with one atomic per workgroup and counter; no normal ever leaves the
+// chip.
 #include <mutex>
 
 #include "mcr_kern_common.h"

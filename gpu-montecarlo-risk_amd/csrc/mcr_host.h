@@ -115,7 +115,7 @@ int fetch_windows(const std::vector<WindowFetch>& w, float** hbuf, size_t* hcap,
 int run_locked(const mcr_query* q, mcr_result* r, bool noalloc = false);
 void set_windows(const mcr_query* q, int n_alpha, FactorArgs* f);
 
-// Persistent batch classes: queries with n <= kSmallMaxN run the per-wave
+// Persistent batch classes: queries with n <= kSmallMaxN run the
 // register-operand MFMA kernel of their (NB, T), larger ones the LDS MFMA
 // kernel of their shape.  Items of one class are contiguous and launched
 // together.

@@ -168,10 +168,11 @@ struct BatchArgs {
   unsigned* next;           // the class's work counter, cleared by k_batch_clear
 };
 
-// Persistent batch kernels, one per class: n <= 127 runs the register-operand
-// MFMA code per wave (class = Philox blocks NB, tiles T); larger n runs the
-// LDS MFMA code per workgroup (class = the workgroup shape chosen for T: waves
-// per workgroup and row-tile slots per wave).
+// Persistent batch kernels, one per class, whose workgroups take the items: n <= 127
+// runs the register-operand MFMA code, an item's groups dealt to the workgroup's
+// four waves (class = Philox blocks NB, tiles T); larger n runs the LDS MFMA code,
+// a group at a time (class = the workgroup shape chosen for T: waves per workgroup
+// and row-tile slots per wave).
 typedef void (*BatchKernel)(BatchArgs);
 BatchKernel batch_small_kernel(int n, int T);  // n <= 127, 256 threads
 int big_waves(int T);                          // waves per workgroup, single-query LDS MFMA kernel

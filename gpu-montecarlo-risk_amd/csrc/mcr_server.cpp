@@ -13,9 +13,9 @@
 //
 // Device work per round r (parity p = r & 1), on two default-priority streams
 // (plus the class-launch forks):
-//   setup:  H2D of new queries' inputs and descriptors, k_factor_batch
-//           (factorisation skipped on a cache hit), k_prep_batch, H2D of the round's work
-//           items; event setup[p].  Overlaps the previous round's path kernel.
+//   setup:  H2D of new queries' inputs and descriptors, k_chol_step_batch
+//           (factorisation skipped on a cache hit), k_factor_batch, k_prep_batch, H2D
+//           of the round's work items; event setup[p].  Overlaps the previous round's path kernel.
 //   paths:  wait setup[p]; k_batch_clear; one persistent launch per kernel class
 //           over the round's items (k_batch_small / k_batch_stage / k_batch_spec),
 //           the classes forked over nfork streams and joined back; events

@@ -12,8 +12,9 @@ namespace mcr {
 // steps (4 KiB a step), and behind a barrier every wave runs its one or two row
 // tiles through, fragments streamed from L2 two steps ahead.  Two or four
 // workgroups per CU, so that one's normals run beside another's products.  Bound:
-// vector issue of the normals, then the matrix instructions not hidden beside
-// them.  Queries of 4e11 / (n^2 + 40 n) paths, against waves that generate and
+// the two units' work, which overlaps little: of the SIMD cycles at n = 143 / 301 /
+// 400 the vector unit issues in 76 / 65 / 63 %, the matrix unit is busy in 22 / 34 /
+// 40, both at once in 12 / 10 / 14, neither in 14 / 11 / 10.  Queries of 4e11 / (n^2 + 40 n) paths, against waves that generate and
 // multiply in turn (n < 384) or take a role each: n = 143 3.16 -> 2.88 ms, n = 200
 // 2.58 -> 2.46, n = 301 2.18 -> 1.99, n = 400 2.18 -> 1.81, n = 511 1.96 -> 1.71.
 // Past 16 row tiles a CU holds one such workgroup, nothing runs beside it, and
@@ -150,8 +151,8 @@ __device__ __forceinline__ void stage_groups(const PathArgs& a, uint64_t g0, uin
       }
       __syncthreads();
       // products before another workgroup's normals: they fill the matrix unit
-      // from few issue slots (1e12 / (n^2 + 40 n) paths, n = 143 7.21 -> 7.12 ms,
-      // n = 400 4.15 -> 4.07, n = 511 3.69 -> 3.60; n = 200 and 301 the same)
+      // from few issue slots (1e12 / (n^2 + 40 n) paths: n = 143, 200 and 255 the
+      // same, n = 301 4.85 -> 4.89 ms, n = 400 4.35 -> 4.23, n = 511 3.79 -> 3.71)
       __builtin_amdgcn_s_setprio(2);
       stage_run<0>(acc, tile, S, sc, min(end0, se), zs + lane, rs, 32 * lane);
       const int s1 = max(sc, end0);

@@ -24,8 +24,9 @@ namespace mcr {
 // D[row][path]: lane l holds rows 8(r/4) + 4(l/32) + r%4 of its column; two
 // more swaps bring the counts and the loss back to the path's lane.
 // Bound: the fp32 matrix instructions (64 cycles for 2 x 32 x 32 multiply-adds)
-// and the vector instructions do not overlap on a SIMD (measured: their times
-// add), so a group costs both in full: at n = 127 320 of the former and 32
+// and the vector instructions do not overlap on a SIMD (counted: no cycle with
+// both, at n = 100 55 % with the former and 40 % with the latter), so a group costs
+// both in full: at n = 127 320 of the former and 32
 // blocks of normals; 4.62 ms for 1.9e7 paths, 8.76 ms in the tile kernel.
 // ---------------------------------------------------------------------------
 template <int T>

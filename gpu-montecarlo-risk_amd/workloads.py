@@ -28,7 +28,7 @@ LARGE_N600 = {"name": "large_n600_10M", "n": 600, "factors": 20, "days": 2500,
 WIDEST_MFMA_N767 = {"name": "widest_mfma_n767_1M", "n": 767, "factors": 20, "days": 4000,
                     "paths": 1_000_000, "k": 10, "x": 0.02, "alphas": (0.99,),
                     "data_seed": 1007, "path_seed": 20251205}
-# Past the LDS MFMA kernel's 767 assets: the column-chunk fp32 kernel.
+# Past the LDS MFMA kernel's 767 assets: the fp32 LDS kernel, in column chunks.
 LARGEST_N1024 = {"name": "largest_n1024_1M", "n": 1024, "factors": 20, "days": 4000,
                  "paths": 1_000_000, "k": 10, "x": 0.02, "alphas": (0.99,),
                  "data_seed": 1006, "path_seed": 20251204}
