@@ -27,22 +27,22 @@ PEAK_BF16_TFLOPS = 2500.0   # MI355X published dense bf16 MFMA
 # HBM bytes per launch of the headline path kernel, from two rocprofv3 --pmc
 # runs of this bench (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 KiB, the factors
 # read off a 256 MiB torch.neg calibration kernel in the same runs).
-TRAFFIC_BYTES = {"mfma": (191.5 * 2.000 + 834.7) * 1024}
+TRAFFIC_BYTES = {"mfma": (1245.2 * 2.000 + 4865.3) * 1024}
 # VALU figures of the headline path kernel from a rocprofv3 --pmc run of this
 # bench (SQ_INSTS_VALU, SQ_ACTIVE_INST_VALU2, SQ_VALU_MFMA_BUSY_CYCLES over
 # GRBM_GUI_ACTIVE, 1024 SIMDs): the unit that binds it is the VALU issue of
 # normal generation (Philox4x32-10, Box-Muller), not the matrix cores.
-VALU_PROFILE = {"mfma": {"valu_lane_instr_per_path": 2509,
-                         "valu_instr_per_simd_quad_cycle": 1.19,
-                         "valu_issue_quad_cycle_frac": 0.914,
-                         "mfma_busy_frac": 0.137,
+VALU_PROFILE = {"mfma": {"valu_lane_instr_per_path": 2245,
+                         "valu_instr_per_simd_quad_cycle": 1.24,
+                         "valu_issue_quad_cycle_frac": 0.900,
+                         "mfma_busy_frac": 0.159,
                          "source": "profiles/k_mfma_n50_100M.md"}}
 # The same figures for the n = 600 split kernel (k_mfma_spec<8,3,4>): VALU
-# issue 0.67 instructions per quad-cycle against its normal-generation bound of
-# one, MFMA busy 40 %.
-LARGE_PROFILE = {"mfma_lds": {"valu_instr_per_simd_quad_cycle": 0.67,
-                              "valu_issue_frac_of_generation_bound": 0.67,
-                              "mfma_busy_frac": 0.40,
+# issue 0.62 instructions per quad-cycle against its normal-generation bound of
+# one, MFMA busy 41 %.
+LARGE_PROFILE = {"mfma_lds": {"valu_instr_per_simd_quad_cycle": 0.62,
+                              "valu_issue_frac_of_generation_bound": 0.62,
+                              "mfma_busy_frac": 0.41,
                               "source": "profiles/k_mfma_spec_n600_10M.md"}}
 
 
@@ -311,7 +311,7 @@ def serve_leg(mcr, np, wl, count, rates):
 
 
 def large_leg(mcr, np, wl):
-    """n = 600, 1e7 paths: plain fp32 tile kernel vs bf16x3 MFMA, same stream."""
+    """n = 600, 1e7 paths: fp32 LDS kernel vs bf16x3 MFMA, same stream."""
     G = wl.LARGE_N600
     mu, sigma = wl.model_of(mcr, G)
     res = {"workload": G["name"], "n_assets": G["n"], "paths": G["paths"],
@@ -335,7 +335,7 @@ def large_leg(mcr, np, wl):
                      "ci": [t.ci_lower, t.ci_upper], "kernel_ms": t.ms_kernel,
                      "count_equals_histogram_tail": t.count == int(h.s_hist[kt:].sum())}
     # the LDS MFMA kernel at its 24 row tiles (bf16x3) and, past 767 assets,
-    # the column-chunk fp32 kernel that every precision then runs
+    # the fp32 LDS kernel that every precision then runs
     W = wl.WIDEST_MFMA_N767
     muw, sigw = wl.model_of(mcr, W)
     wr = [mcr.run(muw, sigw, W["x"], W["k"], W["paths"], W["path_seed"],
@@ -476,13 +476,13 @@ def main():
     extra["fp32_count"] = fnear.count
     extra["fp32_near_threshold"] = fnear.near_threshold
     extra["speedup_vs_fp32_kernel"] = extra["fp32_kernel_ms"] / k_ms
-    roof = {"bound": "mfma" if is_mfma else "valu", "achieved": achieved, "peak": peak,
+    roof = {"bound": "valu", "achieved": achieved, "peak": peak,
             "unit": "TFLOP/s", "frac": achieved / peak,
             "traffic": TRAFFIC_BYTES.get(r.kernel), "kernel": r.kernel, "kernel_ms": k_ms,
             "flop_per_path": n * (n + 1),
-            "note": ("achieved counts the mat-vec FLOPs only; the kernel is bound by the VALU "
-                     "issue of normal generation (Philox4x32-10, Box-Muller), which valu "
-                     "gives from rocprof counters")}
+            "note": ("achieved counts the mat-vec FLOPs only, against the peak of the unit they "
+                     "run on; the kernel is bound by the VALU issue of normal generation "
+                     "(Philox4x32-10, Box-Muller), which valu gives from rocprof counters")}
     if VALU_PROFILE.get(r.kernel):
         roof["valu"] = VALU_PROFILE[r.kernel]
     out = {
